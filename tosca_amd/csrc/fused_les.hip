@@ -91,7 +91,7 @@ template <> struct DsmSum<float> { using type = float; };
 template <class T, class MT = double>
 __global__ void __launch_bounds__(64 * DSM_NR) k_dsm_lm(Geo g, const T *ucat, const MT *csi,
                                                         const MT *eta, const MT *zet, const double *aj,
-                                                        double *LM, double *MM, double *Sabs, int kchunk) {
+                                                        double *LM, double *MM, double *Sabs, int kref, int kchunk) {
     using S = typename DsmSum<T>::type;
     constexpr bool shifted = !std::is_same<S, double>::value;
     __shared__ T sU[3][DSM_NR][64];            // ucat of the plane, for the j neighbours
@@ -100,14 +100,17 @@ __global__ void __launch_bounds__(64 * DSM_NR) k_dsm_lm(Geo g, const T *ucat, co
     const int tile = xcd_tile();                // j fastest, then i, then the k chunk
     const int bj = tile % gridDim.y, bi = (tile / gridDim.y) % gridDim.x, bk = tile / (gridDim.x * gridDim.y);
     const int i = bi * DSM_TI + lane, j = bj * DSM_TJ + r;     // this thread's point column
-    const int kb = 1 + bk * kchunk, ke = min(kb + kchunk, g.mz - 1);   // output planes [kb, ke)
+    // output planes [kb, ke): a piece of kchunk planes of the kref planes from ks on
+    const int np = (kref + kchunk - 1) / kchunk, ks = 1 + (bk / np) * kref, kb = ks + (bk % np) * kchunk;
+    const int ke = min(min(kb + kchunk, ks + kref), g.mz - 1);
+    if (kb >= ke) return;                       // uniform: the last planes have fewer pieces
     // L_ij = <U_i u_j> - <U_i><u_j> is unchanged when U_i and u_j are shifted by constants (the
-    // filter is normalised), so with FP32 sums every point of the tile's march takes the velocity and
-    // the contravariant velocity of one interior cell of the tile out of the two factors
+    // filter is normalised), so with FP32 sums every point of the tile's kref planes takes the velocity
+    // and the contravariant velocity of one interior cell of the tile out of the two factors
     Vec3<T> uref{T(0), T(0), T(0)}, Uref{T(0), T(0), T(0)};
     if constexpr (shifted) {
         const int ic = min(max(bi * DSM_TI + 32, 1), g.mx - 2), jc = min(max(bj * DSM_TJ + 3, 1), g.my - 2);
-        const int kc = min(kb, g.mz - 2);
+        const int kc = min(ks, g.mz - 2);
         tile_shift(ucat, csi, eta, zet, g.L(kc, jc, ic), uref, Uref);
     }
     const bool mi = i >= 1 && i <= g.mx - 2, mj = j >= 1 && j <= g.my - 2;
@@ -730,14 +733,6 @@ void zero_outside_interior(T *a, const Geo &g, hipStream_t s) {
 }
 
 namespace {
-// k planes per chunk of a k-marching launch over `tiles` column tiles: about `target` workgroups in
-// all, at least 8 planes per chunk
-int plane_chunk(int nk, int tiles, int target) {
-    int chunks = (target + tiles - 1) / tiles;
-    chunks = max(1, min(chunks, nk / 8 > 0 ? nk / 8 : 1));
-    return (nk + chunks - 1) / chunks;
-}
-
 // LM, MM (3-point test filter + Germano contraction) and |S| of every interior cell
 // m32: FP32 copies of csi, eta, zet to read instead of the mesh's (FP32 flow fields only)
 template <class T>
@@ -745,17 +740,24 @@ void launch_dsm_lm(const Geo &g, const tosca_mesh *m, const T *ucat, double *LM,
                    const tosca_mesh_f32 *m32 = nullptr) {
     const int nk = g.mz - 2;
     const int ti = (g.mx - 2 + DSM_TI - 1) / DSM_TI, tj = (g.my - 2 + DSM_TJ - 1) / DSM_TJ;
-    const int kchunk = plane_chunk(nk, ti * tj, 2048);
-    dim3 grid(ti, tj, (nk + kchunk - 1) / kchunk);
+    // FP64: chunks as plane_chunk; FP32: pieces of the chunks that share a reference cell (8 planes or
+    // more, about 2048 workgroups), so that the pieces do not change the rounding of the shifted sums
+    int kref = plane_chunk(nk, ti * tj, NUM_CU, 2, 2e4), kchunk = kref;
+    if constexpr (std::is_same<T, float>::value) {
+        const int chunks = max(1, min((2048 + ti * tj - 1) / (ti * tj), nk / 8));
+        kref = (nk + chunks - 1) / chunks;
+        kchunk = plane_chunk(kref, ti * tj * ((nk + kref - 1) / kref), NUM_CU, 2, 2e4);
+    }
+    dim3 grid(ti, tj, ((nk + kref - 1) / kref) * ((kref + kchunk - 1) / kchunk));
     if constexpr (std::is_same<T, float>::value) {
         if (m32) {
             TOSCA_LAUNCH("k_dsm_lm_f32m", (k_dsm_lm<float, float>), grid, dim3(64, DSM_NR), 0, s, g, ucat, m32->csi,
-                         m32->eta, m32->zet, m->aj, LM, MM, Sabs, kchunk);
+                         m32->eta, m32->zet, m->aj, LM, MM, Sabs, kref, kchunk);
             return;
         }
     }
     TOSCA_LAUNCH(sizeof(T) == 8 ? "k_dsm_lm" : "k_dsm_lm_f32", k_dsm_lm<T>, grid, dim3(64, DSM_NR), 0, s, g, ucat, m->csi,
-                 m->eta, m->zet, m->aj, LM, MM, Sabs, kchunk);
+                 m->eta, m->zet, m->aj, LM, MM, Sabs, kref, kchunk);
 }
 
 // launch shape of k_dpasd_k, which sizes the partials buffer
@@ -765,7 +767,7 @@ DpasdK dpasd_k_shape(const Geo &g) {
     const int nk = g.mz - 2;
     d.ti = (g.mx - 2 + DK_X - 1) / DK_X;
     d.tj = (g.my - 2 + DK_Y - 1) / DK_Y;
-    d.kchunk = plane_chunk(nk, d.ti * d.tj, 4096);
+    d.kchunk = plane_chunk(nk, d.ti * d.tj, 4 * NUM_CU, 2, 500.0);
     d.chunks = (nk + d.kchunk - 1) / d.kchunk;
     return d;
 }
@@ -791,7 +793,7 @@ void fused_dpasd(const Geo &g, const tosca_mesh *m, const T *ucat, double maxCs,
     launch_dsm_lm<T>(g, m, ucat, LM, MM, Sabs, s);
     const int nk = g.mz - 2;
     const int ti = (g.mx - 2 + DP_TI - 1) / DP_TI, tj = (g.my - 2 + DP_TJ - 1) / DP_TJ;
-    const int kchunk = plane_chunk(nk, ti * tj, 1536);
+    const int kchunk = plane_chunk(nk, ti * tj, NUM_CU, 1, 2000.0);
     TOSCA_LAUNCH(sizeof(T) == 8 ? "k_dpasd_ij" : "k_dpasd_ij_f32", k_dpasd_ij<T>, dim3(ti, tj, (nk + kchunk - 1) / kchunk),
                  dim3(64, DP_NR), 0, s, g, ucat, m->csi, m->eta, m->zet, m->aj, X, nI, kchunk);
     TOSCA_LAUNCH(sizeof(T) == 8 ? "k_dpasd_k" : "k_dpasd_k_f32", k_dpasd_k<T>, dim3(d.ti, d.tj, d.chunks), dim3(DK_X, DK_Y),
@@ -810,9 +812,7 @@ void fused_dsm(const Geo &g, const tosca_mesh *m, const T *ucat, double maxCs, d
     const int nk = g.mz - 2;
     launch_dsm_lm<T>(g, m, ucat, LM, MM, Sabs, s, m32);
     const int ctiles = ((g.mx - 2 + CX - 1) / CX) * ((g.my - 2 + CY - 1) / CY);
-    int cchunks = max(1, min((2304 + ctiles - 1) / ctiles, nk / 8 > 0 ? nk / 8 : 1));
-    const int ckchunk = (nk + cchunks - 1) / cchunks;
-    cchunks = (nk + ckchunk - 1) / ckchunk;
+    const int ckchunk = plane_chunk(nk, ctiles, 2 * NUM_CU, 2, 500.0), cchunks = (nk + ckchunk - 1) / ckchunk;
     TOSCA_LAUNCH(sizeof(T) == 8 ? "k_dsm_cs_nut" : "k_dsm_cs_nut_f32", k_dsm_cs_nut<T>,
                  dim3((g.mx - 2 + CX - 1) / CX, (g.my - 2 + CY - 1) / CY, cchunks), dim3(CX, CY), 0, s, g, LM, MM, Sabs,
                  m->aj, maxCs, cs, nut, ckchunk);
