@@ -35,7 +35,7 @@ KERNEL_BYTES = {
     # FormU + Buoyancy: ucont, ucat, nut, face metrics, face Jacobians, cell metrics, theta,
     # rhs (+=, read and written), bTheta (written)
     "k_fused_formu": 24 + 24 + 8 + 216 + 24 + 72 + 8 + 2 * 24 + 24,      # = 448
-    "k_dsm_lm": 24 + 72 + 8 + 3 * 8,                      # ucat, cell metrics, aj -> LM, MM, |S|
+    "k_les_filter3": 24 + 72 + 8 + 3 * 8,                 # ucat, cell metrics, aj -> LM, MM, |S|
     "k_dsm_cs_nut": 3 * 8 + 8 + 2 * 8,                    # LM, MM, |S|, aj -> Cs, nut
     "k_nut_fused": 24 + 72 + 8 + 8 + 8,                   # ucat, cell metrics, aj, Cs -> nut
     # reference-structured path
@@ -47,10 +47,9 @@ KERNEL_BYTES = {
     "k_box_clip": 16 + 8 + 8,                             # LM, MM, aj -> Cs
     "k_nut": 24 + 72 + 8 + 8 + 8,                         # ucat, cell metrics, aj, Cs -> nut
     "k_buoyancy": 8 + 72 + 24,                            # theta, icsi/jeta/kzet -> bTheta
-    # plane-averaged dynamic model (DPASD), fused: the 5-point filter's 28 (i, j)-filtered sums
-    # pass through HBM once (written by k_dpasd_ij, read by k_dpasd_k)
-    "k_dpasd_ij": 24 + 72 + 8 + 28 * 8,                   # ucat, cell metrics, aj -> 28 sums
-    "k_dpasd_k": 28 * 8 + 2 * 8 + 72 + 8,                 # 28 sums, LM, MM, cell metrics, aj -> plane partials
+    # plane-averaged dynamic model (DPASD); in FP32 the 5-point filter's 28 (i, j)-filtered sums
+    # pass through HBM once (written by k_dpasd_ij_f32, read by k_dpasd_k_f32)
+    "k_les_filter5": 24 + 72 + 8,                         # ucat, cell metrics, aj -> plane partials
     "k_dpasd_cs_nut": 8 + 8 + 2 * 8,                      # |S|, aj -> Cs, nut
     "k_dpasd_ij_f32": 12 + 72 + 8 + 28 * 4,
     "k_dpasd_k_f32": 28 * 4 + 2 * 8 + 72 + 8,
@@ -349,7 +348,7 @@ def dpasd_leg(torch, ctx, mesh, case, ucont, ucat, theta, lay, args, farm=None):
     for name, fn in (("fp64", fp64), ("mixed", mixed)):
         ms, kms = timed(fn, args.steps)
         rates = {k: KERNEL_BYTES[k] * lay.ncells / (v * 1e-3) / 1e9 for k, v in kms.items()
-                 if k.startswith("k_dpasd") and k in KERNEL_BYTES}
+                 if k.startswith(("k_dpasd", "k_les")) and k in KERNEL_BYTES}
         out[name] = {"ms_per_step": ms, "value": lay.ncells / (ms * 1e-3), "unit": "cell-updates/s",
                      "kernels_ms": kms, "algorithmic_GBs": rates,
                      "frac_of_hbm_peak": {k: v / HBM_PEAK_GBS for k, v in rates.items()}}

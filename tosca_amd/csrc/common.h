@@ -369,6 +369,12 @@ __device__ __forceinline__ int opaque_index(int x) {
     return x;
 }
 
+// The same for a value: its computation is neither repeated nor moved past this point.
+template <class S> __device__ __forceinline__ S opaque_value(S x) {
+    __asm__ volatile("" : "+v"(x));
+    return x;
+}
+
 // Neighbour values across the lanes of a 64-wide wave: shup gives lane l the value of lane l-1,
 // shdn that of lane l+1.  Lane 0 (shup) and lane 63 (shdn) have no neighbour and receive 0; the
 // tiled kernels use both lanes as halo lanes whose own results are discarded.  The DPP wavefront
