@@ -978,7 +978,7 @@ int tosca_ueqn_rk3w_adjoint(tosca_ctx *c, const tosca_mesh *m, const tosca_param
     if (ucont_bar == rhs || ucont_bar == rhs_o || ucont_bar == ucont_o)
         return set_err(c, TOSCA_ERR_ARG, "ucont_bar must not alias the work vectors");
     // the FormU adjoint's workspace, then the checkpoints (n_stages + 1 states) and the work vectors
-    if ((rc = ensure_ws(c, std::max(ws_need(c, p), 52 * n + 64)))) return rc;
+    if ((rc = ensure_ws(c, std::max(ws_need(c, p), tosca::vjp_ws_doubles(g) + 64)))) return rc;
     const size_t need = ((size_t)n_stages + 1) * ng3 + 2 * ng3 + 9 * n;
     if (c->adj_elems < need) {
         if (c->adj) { hipStreamSynchronize(c->stream); hipFree(c->adj); c->adj = nullptr; c->adj_elems = 0; }
@@ -1700,7 +1700,7 @@ int tosca_rhs_vjp(tosca_ctx *c, const tosca_mesh *m, const tosca_params *p, cons
         (rc = check_dev(c, cs_bar, n * sizeof(double), "cs_bar")))
         return rc;
     // nu_t, fpbar, the nu_eff cotangents and the ucat-cotangent packets of the faces and cells
-    if ((rc = ensure_ws(c, std::max(ws_need(c, p), 52 * n + 64)))) return rc;
+    if ((rc = ensure_ws(c, std::max(ws_need(c, p), tosca::vjp_ws_doubles(g) + 64)))) return rc;
     tosca::vjp_rhs(g, m, p, ucont, ucat, theta, cs, rbar, scale, buoy_scale, ucont_bar, ucat_bar, theta_bar, cs_bar,
                    c->ws, c->stream);
     return launched(c, "rhs_vjp");
@@ -1728,7 +1728,7 @@ int tosca_rhs_vjp_mixed(tosca_ctx *c, const tosca_mesh *m, const tosca_params *p
         (rc = check_dev(c, ucat_bar, v, "ucat_bar")) || (rc = check_dev(c, theta_bar, n * sizeof(float), "theta_bar")) ||
         (rc = check_dev(c, cs_bar, n * sizeof(double), "cs_bar")))
         return rc;
-    if ((rc = ensure_ws(c, std::max(ws_need(c, p), 52 * n + 64)))) return rc;
+    if ((rc = ensure_ws(c, std::max(ws_need(c, p), tosca::vjp_ws_doubles(g) + 64)))) return rc;
     tosca::vjp_rhs_mixed(g, m, p, ucont, ucat, cs, rbar, scale, buoy_scale, ucont_bar, ucat_bar, theta_bar, cs_bar,
                          c->ws, c->stream);
     return launched(c, "rhs_vjp_mixed");

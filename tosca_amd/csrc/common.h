@@ -417,12 +417,13 @@ __device__ __forceinline__ double pmin(double a, double b) { return (a < b) ? a 
 #define TOSCA_XCD_TILES 1
 #endif
 constexpr int NUM_XCD = 8;
-__device__ __forceinline__ int xcd_tile() {
-    const int n = gridDim.x * gridDim.y * gridDim.z;
-    const int w = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+__device__ __forceinline__ int xcd_tile(int w, int n) {
     if (!TOSCA_XCD_TILES) return w;
     const int q = n / NUM_XCD, r = n % NUM_XCD, x = w % NUM_XCD, slot = w / NUM_XCD;
     return (x < r) ? x * (q + 1) + slot : r * (q + 1) + (x - r) * q + slot;
+}
+__device__ __forceinline__ int xcd_tile() {
+    return xcd_tile(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), gridDim.x * gridDim.y * gridDim.z);
 }
 
 }  // namespace tosca

@@ -100,7 +100,8 @@ template <class T>
 void nut_bcs(T *nut, const tosca_params *p, const Geo &g, hipStream_t s);
 
 // Adjoint of R = FormU(ucont, ucat, UpdateNut(ucat, cs)) + Buoyancy(theta): accumulates the
-// cotangents of the four inputs (overwritten) from rbar; ws holds >= 52 * nloc doubles.
+// cotangents of the four inputs (overwritten) from rbar; ws holds vjp_ws_doubles(g) doubles.
+size_t vjp_ws_doubles(const Geo &g);
 void vjp_rhs(const Geo &g, const tosca_mesh *mesh, const tosca_params *p, const double *ucont, const double *ucat,
              const double *theta, const double *cs, const double *rbar, double scale, double buoy_scale,
              double *ucont_bar, double *ucat_bar, double *theta_bar, double *cs_bar, double *ws, hipStream_t s);
@@ -113,7 +114,7 @@ void vjp_rhs_mixed(const Geo &g, const tosca_mesh *mesh, const tosca_params *p, 
                    float *ucat_bar, float *theta_bar, double *cs_bar, double *ws, hipStream_t s);
 
 // Adjoint of FormU(ucont, ucat, nu_t; scale, formMode 0) with nu_t an input: ucont_bar and ucat_bar
-// overwritten, the nu_t cotangent added to nut_bar (LES active); ws holds >= 52 * nloc doubles.
+// overwritten, the nu_t cotangent added to nut_bar (LES active); ws as vjp_rhs.
 void vjp_formu_nut(const Geo &g, const tosca_mesh *mesh, const tosca_params *p, const double *ucont, const double *ucat,
                    const double *nut, const double *rbar, double scale, double *ucont_bar, double *ucat_bar,
                    double *nut_bar, double *ws, hipStream_t s);

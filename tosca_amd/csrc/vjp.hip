@@ -9,18 +9,20 @@
 //   k_vjp_fp      face dot (ueqn_solvers.c:1006-1035) -> fpbar per interior cell (a gather: the
 //                 cell's own faces, the faces of its lower neighbours, and the ghost m-1 aliases:
 //                 cell 1 on a periodic axis, the copied cell m-2 otherwise)
-//   k_vjp_faces   (the i, j and k faces of each index point) cell divergence (ueqn_solvers.c:871-993) -> face-flux cotangent, then the
-//                 convective flux (central / QUICK, inline.h:4314-4324, 5089-5109) -> ucont_bar and
-//                 a packet of ucat cotangents, the viscous flux (ueqn_solvers.c:184-216...) -> the
-//                 cotangents of its nine derivatives (Compute_du_i/j/k, inline.h:2748-2931) into the
-//                 same packet, and the nu_eff cotangent.  Only the boundary faces scatter (atomics).
-//   k_vjp_nut     nu_t = Cs Delta^2 |S| (les.c:2510-2514), with the UpdateNutBCs ghosts
-//                 (boundary.c:2812-2917) transposed -> Cs_bar, and a packet for the |S| path
-//                 (Compute_du_dxyz / Compute_du_center, inline.h:3344-3418, 3635-3663)
-//   k_vjp_gather  per owned point: ucat_bar from the packets of the faces and cells whose regular
-//                 stencils reach it, and theta_bar from Buoyancy (ueqn_sources.c:2812-2870)
+//   k_vjp_march   the interior faces: cell divergence (ueqn_solvers.c:871-993) -> face-flux cotangent, then
+//                 the convective flux (central / QUICK, inline.h:4314-4324, 5089-5109) -> ucont_bar and its
+//                 ucat cotangent, the viscous flux (ueqn_solvers.c:184-216...) -> the cotangents of its nine
+//                 derivatives (Compute_du_i/j/k, inline.h:2748-2931) and of nu_eff; the ucat cotangents
+//                 summed per row of points, marching along k.  The launch's last workgroups take the
+//                 boundary faces, whose stencils are one-sided or clipped: a scatter (atomics)
+//   k_vjp_finish  nu_t = Cs Delta^2 |S| (les.c:2510-2514), with the UpdateNutBCs ghosts
+//                 (boundary.c:2812-2917) transposed -> Cs_bar and the |S| path (Compute_du_dxyz /
+//                 Compute_du_center, inline.h:3344-3418, 3635-3663), added to the row sums -> ucat_bar;
+//                 theta_bar from Buoyancy (ueqn_sources.c:2812-2870).  k_vjp_sum: the row sums alone
 // The forward intermediates the adjoint needs (nu_t, the face gradients, the interpolated face
 // velocities) are recomputed from the inputs instead of being stored by the forward pass.
+#include <type_traits>
+
 #include "fused.h"
 
 namespace tosca {
@@ -125,9 +127,9 @@ struct VjpArgs {
     T *vbar, *ubar, *tbar;
     double *csbar;
     double *nutbar_acc; // nu_t given as an input: its cotangent is accumulated here (local)
-    P *pk[3];           // per face direction: 12 SoA planes of n values (cv, gn, ga, gb)
     P *nueb[3];         // per face direction: cotangent of nu_eff at each face (n values)
-    P *spk;             // per interior cell: 9 SoA planes (cotangents of the du_center derivatives)
+    P *rows;            // ucat cotangents summed per row: own, jp, jm, jpp (k_vjp_march), n vectors each
+    double *tb;         // theta cotangents summed per row: the row's own, row j+1's (n values each)
     long n;
     double scale, bscale, tRef, nu;
     int quick, les;
@@ -153,12 +155,30 @@ __device__ __forceinline__ void stp3(P *p, int c, V3 v) { p[3 * c] = P(v.x); p[3
 template <class P>
 __device__ __forceinline__ V3 ldp3(const P *p, int c) { return V3{double(p[3 * c]), double(p[3 * c + 1]), double(p[3 * c + 2])}; }
 
-template <class T>
-__global__ void k_vjp_zero(T *a, long n) {
-    for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) a[t] = T(0);
-}
-
 }  // namespace
+
+// zeroes the outer layers of several local arrays in one launch: blockIdx.z selects the array (words 4-byte
+// words per point, w layers from either side, ghosts included), blockIdx.y the side
+struct ZeroShells { unsigned *p[8]; int words[8], w[8], n; };
+__global__ void __launch_bounds__(256) k_vjp_zero_shells(ZeroShells Z, Geo g) {
+    const int q = blockIdx.z, side = blockIdx.y, w = Z.w[q], words = Z.words[q];
+    // low / high k slabs over the whole planes, low / high j slabs between them, low / high i slabs between those
+    int i0 = 0, j0 = 0, k0 = 0, ni = g.gxm, nj = g.gym, nk = g.gzm;
+    if (side < 2) { k0 = side ? g.gzm - w : 0; nk = w; }
+    else {
+        k0 = w; nk = g.gzm - 2 * w;
+        if (side < 4) { j0 = side == 3 ? g.gym - w : 0; nj = w; }
+        else { j0 = w; nj = g.gym - 2 * w; i0 = side == 5 ? g.gxm - w : 0; ni = w; }
+    }
+    if (nj <= 0 || nk <= 0) return;
+    // (on an axis shorter than 2 w the two slabs overlap)
+    const int row = ni * words, tot = row * nj * nk;
+    unsigned *p = Z.p[q];
+    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < tot; t += gridDim.x * blockDim.x) {
+        const int e = t % row, l = t / row;
+        p[(((long)(k0 + l / nj) * g.gym + (j0 + l % nj)) * g.gxm + i0) * words + e] = 0u;
+    }
+}
 
 // fpbar of interior cell (i, j, k) (a gather; no atomics); S: its csi, eta, zet
 template <class T, class P>
@@ -227,14 +247,13 @@ __global__ void __launch_bounds__(256) k_vjp_pre(VjpArgs<T, P> A, Geo g) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// Faces: the flux cotangent, ucont_bar, the nu_eff cotangent, and the ucat cotangent packets.
-// Interior faces (1 <= f <= m-3 along the face direction) store a packet -- the convective
-// cotangent cv = -V Fbar and the cotangents of the normal and two transverse derivatives -- that
-// k_vjp_gather later folds into ucat_bar with the regular stencils; the two boundary faces per line
-// (the only ones with the one-sided and clipped stencils) scatter into ucat_bar directly.
-// Thread x runs along i for every face direction (coalesced).
+// The two boundary faces per line (the only ones with the one-sided and clipped stencils): the flux
+// cotangent, ucont_bar, the nu_eff cotangent, and a scatter into ucat_bar.  About 39 atomics a face and
+// three components, at what the L2 takes; the faces run as the last workgroups of the marching launch,
+// where they fill its last wave (the 192 x 192 x 128 hill: 0.06 ms there, 0.13 in a launch of their own,
+// 0.11 as the first workgroups).
 // ------------------------------------------------------------------------------------------------
-// one face of direction DIR: x = (i, j, k) its index point, f = x[DIR] in 0 .. m-2, the other two
+// one face of direction DIR: x = (i, j, k) its index point, f = x[DIR] = 0 or m-2, the other two
 // in 1 .. m-2
 template <int DIR, class T, class P>
 __device__ __forceinline__ void face_adj(const VjpArgs<T, P> &A, const Geo &g, const int *x) {
@@ -245,7 +264,6 @@ __device__ __forceinline__ void face_adj(const VjpArgs<T, P> &A, const Geo &g, c
     const int i = x[0], j = x[1], k = x[2];
     const int c = g.L(k, j, i);
     const int up = (DIR == 0) ? g.L(k, j, i + 1) : (DIR == 1) ? g.L(k, j + 1, i) : g.L(k + 1, j, i);
-    const bool interior = f >= 1 && f <= m[DIR] - 3;
     // cotangent of the face flux: + fp of the left cell, - fp of the right cell (interior cells)
     V3 Fb{0, 0, 0};
     if (f >= 1) Fb = add3v(Fb, ldp3(A.fpbar, c));
@@ -268,16 +286,15 @@ __device__ __forceinline__ void face_adj(const VjpArgs<T, P> &A, const Geo &g, c
         const int cLL = g.L(xl[2], xl[1], xl[0]), cRR = g.L(xr[2], xr[1], xr[0]);
         const V3 uf = cvt3<double>(quick(ld3(u, cLL), ld3(u, c), ld3(u, up), ld3(u, cRR), VT));
         A.vbar[3 * c + DIR] = T(-dot3(Fb, uf));
-        if (!interior) {
-            // d/dfU = 1/2 + 2/8, d/dfD = 1/2 - 1/8, d/dfUU = -1/8
-            if (V > 0) { aadd3(A.ubar, c, sc3(0.75, cv)); aadd3(A.ubar, up, sc3(0.375, cv)); aadd3(A.ubar, cLL, sc3(-0.125, cv)); }
-            else { aadd3(A.ubar, up, sc3(0.75, cv)); aadd3(A.ubar, c, sc3(0.375, cv)); aadd3(A.ubar, cRR, sc3(-0.125, cv)); }
-        }
+        // d/dfU = 1/2 + 2/8, d/dfD = 1/2 - 1/8, d/dfUU = -1/8
+        if (V > 0) { aadd3(A.ubar, c, sc3(0.75, cv)); aadd3(A.ubar, up, sc3(0.375, cv)); aadd3(A.ubar, cLL, sc3(-0.125, cv)); }
+        else { aadd3(A.ubar, up, sc3(0.75, cv)); aadd3(A.ubar, c, sc3(0.375, cv)); aadd3(A.ubar, cRR, sc3(-0.125, cv)); }
     } else {
         const Vec3<T> a0 = ld3(u, c), a1 = ld3(u, up);
         const V3 uf{double(T(0.5) * (a0.x + a1.x)), double(T(0.5) * (a0.y + a1.y)), double(T(0.5) * (a0.z + a1.z))};
         A.vbar[3 * c + DIR] = T(-dot3(Fb, uf));
-        if (!interior) { aadd3(A.ubar, c, sc3(0.5, cv)); aadd3(A.ubar, up, sc3(0.5, cv)); }
+        aadd3(A.ubar, c, sc3(0.5, cv));
+        aadd3(A.ubar, up, sc3(0.5, cv));
     }
     // ---- viscous ------------------------------------------------------------------------------------
     double nuEff = A.nu;
@@ -314,233 +331,422 @@ __device__ __forceinline__ void face_adj(const VjpArgs<T, P> &A, const Geo &g, c
         return V3{gX1 * Fa.x + d * nrm.x, gX1 * Fa.y + d * nrm.y, gX1 * Fa.z + d * nrm.z};
     };
     const V3 gc = gx(g11, fc), ge = gx(g21, fe), gz = gx(g31, fz);
-    if (interior) {
-        // packet: cv, normal, transverse a, transverse b (a/b: the lower / higher other axis)
-        const V3 gn = (DIR == 0) ? gc : (DIR == 1) ? ge : gz;
-        const V3 ga = (DIR == 0) ? ge : gc;
-        const V3 gb = (DIR == 2) ? ge : gz;
-        const V3 pv[4] = {cv, gn, ga, gb};
-        P *pk = A.pk[DIR];
-        for (int w = 0; w < 4; w++) {
-            pk[(3 * w + 0) * A.n + c] = P(pv[w].x);
-            pk[(3 * w + 1) * A.n + c] = P(pv[w].y);
-            pk[(3 * w + 2) * A.n + c] = P(pv[w].z);
-        }
-    } else if (nuEff != 0.0) {
+    if (nuEff != 0.0) {
         if (DIR == 0) du_i_adj(g, A.ubar, i, j, k, gc, ge, gz);
         else if (DIR == 1) du_j_adj(g, A.ubar, i, j, k, gc, ge, gz);
         else du_k_adj(g, A.ubar, i, j, k, gc, ge, gz);
     }
 }
 
-// the i, j and k faces of index point (i, j, k), i in 0 .. mx-2, j in 0 .. my-2, k in 0 .. mz-2
-// (each face where it exists): the three share the point's fpbar, ucont, nu_t and ucat loads
+// thread t of the boundary workgroups: face set t / nmax (direction, low or high side), point t % nmax of it
 template <class T, class P>
-__global__ void __launch_bounds__(256) k_vjp_faces(VjpArgs<T, P> A, Geo g) {
-    const int x[3] = {(int)(blockIdx.x * blockDim.x + threadIdx.x), (int)blockIdx.y, (int)blockIdx.z};
-    if (x[0] > g.mx - 2) return;
-    const bool in0 = x[0] >= 1, in1 = x[1] >= 1, in2 = x[2] >= 1;
-    if (in1 && in2) face_adj<0>(A, g, x);
-    if (in0 && in2) face_adj<1>(A, g, x);
-    if (in0 && in1) face_adj<2>(A, g, x);
+__device__ __forceinline__ void boundary_face(const VjpArgs<T, P> &A, const Geo &g, int t, int nmax) {
+    const int set = t / nmax, d = set / 2, m[3] = {g.mx, g.my, g.mz};
+    if (set >= 6) return;
+    const int n1 = d == 0 ? g.my : g.mx, n2 = d == 2 ? g.my : g.mz;      // transverse sizes, fastest first
+    const int a = t % nmax % n1, b = t % nmax / n1;
+    if (a < 1 || a > n1 - 2 || b < 1 || b > n2 - 2) return;
+    const int f = set % 2 ? m[d] - 2 : 0;
+    const int x[3] = {d == 0 ? f : a, d == 0 ? a : d == 1 ? f : b, d == 2 ? f : b};
+    if (d == 0) face_adj<0>(A, g, x);
+    else if (d == 1) face_adj<1>(A, g, x);
+    else face_adj<2>(A, g, x);
 }
 
 // ------------------------------------------------------------------------------------------------
-// Interior cells: nu_t_bar (gathered from the nu_eff cotangents of the cell's six faces, plus the
-// ghosts UpdateNutBCs fills from this cell), Cs_bar, and the packet of the |S| path.
-// ------------------------------------------------------------------------------------------------
-template <class T, class P>
-__global__ void __launch_bounds__(256) k_vjp_nut(VjpArgs<T, P> A, Geo g) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x + 1, j = blockIdx.y * blockDim.y + threadIdx.y + 1,
-              k = blockIdx.z + 1;
-    if (i > g.mx - 2 || j > g.my - 2 || k > g.mz - 2) return;
-    const int c = g.L(k, j, i);
-    const int x[3] = {i, j, k}, m[3] = {g.mx, g.my, g.mz};
-    double nb = 0.0;
-    for (int q = 0; q < 3; q++) {
-        int t[3] = {i, j, k};
-        nb += 0.5 * double(A.nueb[q][c]);                              // face q of the cell
-        t[q] = x[q] - 1;
-        if (!(x[q] == 1 && g.per[q] != TOSCA_PERIODIC_NONE))          // periodic face 0 is not evaluated
-            nb += 0.5 * double(A.nueb[q][g.L(t[2], t[1], t[0])]);
-        // ghosts filled from this cell: cotangent of nu_t there is 1/2 nu_eff_bar of the boundary face
-        const int bl = A.bc_nut[2 * q], br = A.bc_nut[2 * q + 1];
-        const bool pq = g.per[q] != TOSCA_PERIODIC_NONE;
-        t[q] = 0;                                                      // face 0 (its left cell is ghost 0)
-        const int f0 = g.L(t[2], t[1], t[0]);
-        t[q] = m[q] - 2;                                               // face m-2 (right cell ghost m-1)
-        const int fm = g.L(t[2], t[1], t[0]);
-        if (bl == TOSCA_BCNUT_ZEROGRADIENT && x[q] == 1) nb += 0.5 * double(A.nueb[q][f0]);
-        if (bl == TOSCA_BCNUT_PERIODIC && pq && x[q] == m[q] - 2) nb += 0.5 * double(A.nueb[q][f0]);
-        if (br == TOSCA_BCNUT_ZEROGRADIENT && x[q] == m[q] - 2) nb += 0.5 * double(A.nueb[q][fm]);
-        if (br == TOSCA_BCNUT_PERIODIC && pq && x[q] == 1) nb += 0.5 * double(A.nueb[q][fm]);
+// Interior faces (1 <= f <= m-3 along the face direction), marching along k: ucont_bar, the nu_eff
+// cotangents and the ucat cotangents of their regular stencils.
+//
+// A wave is one row j of 64 points along i and steps through the planes; lane 0 is point i0 - 2, and the
+// 60 lanes 2 .. 61 own their cell (a cell collects from the faces i-2 .. i+1).  Waves are independent
+// (no LDS, no barrier).  Each plane the thread evaluates the i, j and k face of its point: the
+// convective cotangent cv = -V Fbar and the cotangents gc, ge, gz of the three derivative vectors.  A
+// face contributes to the cells
+//   normal derivative        left -gn, right +gn
+//   convective interpolation left and right (QUICK: left 3/4 or 3/8, right 3/8 or 3/4, and -1/8 of the
+//                            cell upwind of the pair)
+//   transverse derivatives   for both cells of the pair: +g/4 one up, -g/4 one down the transverse axis
+// and these are added where they land: along i by lane shifts, along k in the accumulators of four
+// planes, and only what goes to the neighbouring rows leaves the thread: per point the row's own sum
+// `own`, `jp` for row j+1, `jm` for row j-1 and (QUICK) `jpp` for row j+2, 9 or 12 values instead of
+// the 36 of three face packets.  k_vjp_finish adds the rows.  Buoyancy's theta cotangent comes along,
+// since its icsi.z, jeta.z, kzet.z are loaded here.
+//
+// Bound by memory: 504 bytes a point in FP64 (nine metric vectors 216, four arrays of row sums 96), about
+// 890 moved, since a wave's 64 points end within cache lines, 4 of them overlap and a chunk of planes loads 3
+// more.  The registers (two waves a SIMD) hold the sums of four planes; the row sums and ucont_bar are
+// written as whole vectors, since stores of 8 of 24 bytes cost a pass over the line each.  Against a launch
+// that wrote the three packets of every face and a cell kernel that gathered them: the adjoint of the
+// 192 x 192 x 128 hill (FP64, QUICK) 2.60 -> 1.53 ms, of which this kernel is 0.82, and of the 384 x 256 x 96
+// box (mixed, central) 3.69 -> 2.07, of which 1.03.
+template <class T, class P, bool QUICK>
+__global__ void __launch_bounds__(256, 2) k_vjp_march(VjpArgs<T, P> A, Geo g, int kchunk, int ti, int tj, int nbnd, int nmax) {
+    const int lane = threadIdx.x;
+    const int nm = gridDim.x - nbnd;
+    if (blockIdx.x >= nm) {
+        boundary_face(A, g, ((blockIdx.x - nm) * 4 + threadIdx.y) * 64 + lane, nmax);
+        return;
     }
-    const V3 cc = ld3(A.csi, c), ee = ld3(A.eta, c), zz = ld3(A.zet, c);
-    const double a = A.aj[c];
-    // the strain as the forward computes it (in T), the rest in FP64
-    const CartT<T> dT = du_dxyz(cvt3<T>(cc), cvt3<T>(ee), cvt3<T>(zz), T(a), du_center(g, A.ucat, i, j, k));
-    const Cart d{double(dT.du_dx), double(dT.du_dy), double(dT.du_dz), double(dT.dv_dx), double(dT.dv_dy),
-                 double(dT.dv_dz), double(dT.dw_dx), double(dT.dw_dy), double(dT.dw_dz)};
-    const double S = double(strain_mag(dT));
-    const double filter = cube_root(1. / a), d2 = filter * filter;
-    A.csbar[c] = nb * d2 * S;
-    V3 gc{0, 0, 0}, ge{0, 0, 0}, gz{0, 0, 0};
-    if (S != 0.0 && nb != 0.0) {                   // |S| is not differentiable at 0: subgradient 0
-        // d|S| / dD_mn = 2 S_mn / |S|, S = sym(D)
-        const double sb = nb * A.cs[c] * d2 * 2.0 / S;
-        const double Sxx = d.du_dx, Sxy = 0.5 * (d.du_dy + d.dv_dx), Sxz = 0.5 * (d.du_dz + d.dw_dx);
-        const double Syy = d.dv_dy, Syz = 0.5 * (d.dv_dz + d.dw_dy), Szz = d.dw_dz;
-        const V3 Du{sb * Sxx, sb * Sxy, sb * Sxz}, Dv{sb * Sxy, sb * Syy, sb * Syz}, Dw{sb * Sxz, sb * Syz, sb * Szz};
-        // D_m. = aj (d_c u_m csi + d_e u_m eta + d_z u_m zet)  ->  d_X u_m bar = aj (Dbar_m . M_X)
-        gc = V3{a * dot3(Du, cc), a * dot3(Dv, cc), a * dot3(Dw, cc)};
-        ge = V3{a * dot3(Du, ee), a * dot3(Dv, ee), a * dot3(Dw, ee)};
-        gz = V3{a * dot3(Du, zz), a * dot3(Dv, zz), a * dot3(Dw, zz)};
-    }
-    const V3 pv[3] = {gc, ge, gz};
-    for (int w = 0; w < 3; w++) {
-        A.spk[(3 * w + 0) * A.n + c] = P(pv[w].x);
-        A.spk[(3 * w + 1) * A.n + c] = P(pv[w].y);
-        A.spk[(3 * w + 2) * A.n + c] = P(pv[w].z);
+    const int tile = xcd_tile(blockIdx.x, nm);      // j fastest, then i, then the k chunk
+    const int bj = tile % tj, bi = (tile / tj) % ti, bk = tile / (ti * tj);
+    const int j = 1 + bj * 4 + threadIdx.y, i = bi * 60 + lane - 2;
+    if (j > g.my - 2) return;                          // whole waves; the kernel has no barrier
+    const int kb = bk * kchunk, ke = min(kb + kchunk, g.mz);     // cells [kb, ke)
+    const int ia = min(max(i, 0), g.mx - 1);
+    const int SJ = g.gxm, SK = g.gxm * g.gym, c0 = g.L(0, j, ia);
+    const bool mine = lane >= 2 && lane < 62 && i < g.mx;
+    const bool cellI = i >= 1 && i <= g.mx - 2;
+    const bool okJ0 = cellI && j <= g.my - 3;
+    const long n = A.n;
+    P *own = A.rows, *jp = A.rows + 3 * n, *jm = A.rows + 6 * n, *jpp = A.rows + 9 * n;
+    auto up = [](V3 v) { return shup3(v); };           // the value of lane - 1
+    auto dn = [](V3 v) { return shdn3(v); };           // the value of lane + 1
+    auto sel = [](bool ok, V3 v) { return V3{ok ? v.x : 0.0, ok ? v.y : 0.0, ok ? v.z : 0.0}; };
+    const V3 Z{0, 0, 0};
+    // sums of the cells of planes t-1 .. t+2 of this row, of planes t-1 .. t+1 for row j+1, the k face's
+    // transverse-j cotangent of plane t-1, and the k face's theta cotangent of plane t-1
+    V3 a0 = Z, a1 = Z, a2 = Z, a3 = Z, p0 = Z, p1 = Z, p2 = Z, tk = Z;
+    double hk = 0.0;
+    for (int t = kb - 2; t <= ke; t++) {
+        const int tc = min(max(t, 0), g.mz - 1);
+        const int c = opaque_index(c0 + tc * SK);
+        const bool cell = cellI && t >= 1 && t <= g.mz - 2;      // an interior cell (its + faces exist)
+        const bool face = t >= kb && t < ke && mine;             // this thread's faces are written
+        const bool okI = cell && i <= g.mx - 3, okJ = cell && okJ0, okK = cell && t <= g.mz - 3;
+        const V3 fb = ldp3(A.fpbar, c), fbj = ldp3(A.fpbar, c + SJ), fbk = ldp3(A.fpbar, c + SK), fbi = dn(fb);
+        T n0 = T(0), nj = T(0), nk = T(0), ni = T(0);
+        if (A.les) { n0 = A.nut[c]; nj = A.nut[c + SJ]; nk = A.nut[c + SK]; ni = shdn(n0); }
+        const Vec3<T> V = ld3(A.ucont, c);
+        const Vec3<T> u = ld3(A.ucat, c), uj = ld3(A.ucat, c + SJ), ujm = ld3(A.ucat, c - SJ), uk = ld3(A.ucat, c + SK),
+                      ukm = ld3(A.ucat, c - SK);
+        // (lane shifts stay outside the branches: they read lanes that may not take them)
+        const Vec3<T> ui = shdn3(u), uii = shdn3(ui), uim = shup3(u), uji = shdn3(uj), uki = shdn3(uk);
+        const T q4 = T(0.25);
+        auto four = [&](Vec3<T> a, Vec3<T> b, Vec3<T> m, Vec3<T> o) {
+            return V3{double((a.x + b.x - m.x - o.x) * q4), double((a.y + b.y - m.y - o.y) * q4),
+                      double((a.z + b.z - m.z - o.z) * q4)};
+        };
+        auto diff = [&](Vec3<T> a, Vec3<T> b) { return V3{double(a.x - b.x), double(a.y - b.y), double(a.z - b.z)}; };
+        // one face: flux cotangent F, normal flux W, derivative vectors d[0..2], face metrics; returns the
+        // nu_eff cotangent and writes cv and the cotangents G of the three derivative vectors
+        auto adj = [&](auto dir, bool ok, V3 F, double W, const V3 (&d)[3], double nuEff, V3 fc, V3 fe, V3 fz, double ajc, V3 &cv,
+                       V3 (&G)[3]) {
+            constexpr int DIR = decltype(dir)::value;
+            cv = sc3(-W, F);
+            double nb = 0.0;
+            if (A.les) {
+                const Grad gr{d[0].x, d[0].y, d[0].z, d[1].x, d[1].y, d[1].z, d[2].x, d[2].y, d[2].z};
+                nb = dot3(F, visc_flux(gr, fc, fe, fz, DIR, ajc, 1.0));
+            }
+            // visc_m = a nu (g_X1 d_X u_m + (M_X . d_X u) n_m) summed over X = csi, eta, zet
+            const V3 M[3] = {fc, fe, fz};
+            const V3 nrm = M[DIR], Fa = sc3(ok ? ajc * nuEff : 0.0, F);
+#pragma unroll
+            for (int X = 0; X < 3; X++) {
+                const double gX = dot3(M[X], nrm), s = dot3(M[X], Fa);
+                G[X] = sel(ok, V3{gX * Fa.x + s * nrm.x, gX * Fa.y + s * nrm.y, gX * Fa.z + s * nrm.z});
+            }
+            return ok ? nb : 0.0;
+        };
+        // face value of u for ucont_bar, and the weights of the left and right cell and (QUICK) the cells beyond
+        auto face_u = [&](Vec3<T> m1, Vec3<T> l, Vec3<T> r, Vec3<T> r2, T W) {
+            if constexpr (QUICK) return cvt3<double>(quick(m1, l, r, r2, W));
+            const T h = T(0.5);
+            return V3{double(h * (l.x + r.x)), double(h * (l.y + r.y)), double(h * (l.z + r.z))};
+        };
+        V3 cv, G[3], vb = Z;
+        const double w = A.bscale * (9.81 * 0.5) / A.tRef;
+        double rb[3] = {0, 0, 0};
+        if (A.tbar && cell) { const int gi = 3 * g.G(t, j, i); rb[0] = A.rbar[gi]; rb[1] = A.rbar[gi + 1]; rb[2] = A.rbar[gi + 2]; }
+        V3 T0 = tk;                                    // to rows j+1 (+) and j-1 (-), plane t
+        double h = hk, hj = 0.0;
+        // ---- i face ---------------------------------------------------------------------------------
+        {
+            const T W = okI ? V.x : T(0);            // (what a face that is not evaluated here holds stays out)
+            const V3 fc = ld3(A.icsi, c), fe = ld3(A.ieta, c), fz = ld3(A.izet, c);
+            const V3 d[3] = {diff(ui, u), four(uji, uj, shdn3(ujm), ujm), four(uki, uk, shdn3(ukm), ukm)};
+            const double nuEff = A.les ? A.nu + 0.5 * (double(n0) + double(ni)) : A.nu;
+            const V3 F = sel(okI, add3v(fb, sc3(-1.0, fbi)));
+            vb.x = opaque_value(okI ? -dot3(F, face_u(uim, u, ui, uii, W)) : 0.0);
+            const double nb = adj(std::integral_constant<int, 0>(), okI, F, double(W), d, nuEff, fc, fe, fz, A.iaj[c], cv, G);
+            if (face && okI) A.nueb[0][c] = P(nb);
+            const bool pos = W > T(0);
+            const double wl = QUICK ? (pos ? 0.75 : 0.375) : 0.5, wr = QUICK ? (pos ? 0.375 : 0.75) : 0.5;
+            V3 r = add3v(sc3(wr, cv), G[0]);
+            if constexpr (QUICK) {
+                r = add3v(r, up(sc3(pos ? 0.0 : -0.125, cv)));
+                a1 = add3v(a1, dn(sc3(pos ? -0.125 : 0.0, cv)));
+            }
+            a1 = add3v(a1, add3v(add3v(sc3(wl, cv), sc3(-1.0, G[0])), up(r)));
+            T0 = add3v(T0, sc3(0.25, add3v(G[1], up(G[1]))));
+            const V3 b = sc3(0.25, add3v(G[2], up(G[2])));
+            a2 = add3v(a2, b);
+            a0 = add3v(a0, sc3(-1.0, b));
+            const double hi = cell ? w * fc.z * rb[0] : 0.0;
+            h += hi + shup(hi);
+        }
+        V3 JM = Z;
+        // ---- j face ---------------------------------------------------------------------------------
+        {
+            const T W = okJ ? V.y : T(0);            // (what a face that is not evaluated holds stays out)
+            const V3 fc = ld3(A.jcsi, c), fe = ld3(A.jeta, c), fz = ld3(A.jzet, c);
+            const V3 d[3] = {four(uji, ui, shup3(uj), uim), diff(uj, u),
+                             four(ld3(A.ucat, c + SK + SJ), uk, ld3(A.ucat, c - SK + SJ), ukm)};
+            const double nuEff = A.les ? A.nu + 0.5 * (double(n0) + double(nj)) : A.nu;
+            const V3 F = sel(okJ, add3v(fb, sc3(-1.0, fbj)));
+            Vec3<T> ujj = uj;
+            if constexpr (QUICK) ujj = ld3(A.ucat, c + 2 * SJ);
+            vb.y = opaque_value(okJ ? -dot3(F, face_u(ujm, u, uj, ujj, W)) : 0.0);
+            const double nb = adj(std::integral_constant<int, 1>(), okJ, F, double(W), d, nuEff, fc, fe, fz, A.jaj[c], cv, G);
+            if (face && okJ) A.nueb[1][c] = P(nb);
+            const bool pos = W > T(0);
+            const double wl = QUICK ? (pos ? 0.75 : 0.375) : 0.5, wr = QUICK ? (pos ? 0.375 : 0.75) : 0.5;
+            const V3 ld = sc3(0.25, add3v(up(G[0]), sc3(-1.0, dn(G[0]))));
+            a1 = add3v(a1, add3v(add3v(sc3(wl, cv), sc3(-1.0, G[1])), ld));
+            p1 = add3v(p1, add3v(add3v(sc3(wr, cv), G[1]), ld));
+            if constexpr (QUICK) {
+                JM = sc3(pos ? -0.125 : 0.0, cv);
+                if (face) stp3(jpp, c, sc3(pos ? 0.0 : -0.125, cv));
+            }
+            const V3 b = sc3(0.25, G[2]);
+            a2 = add3v(a2, b);
+            a0 = add3v(a0, sc3(-1.0, b));
+            p2 = add3v(p2, b);
+            p0 = add3v(p0, sc3(-1.0, b));
+            hj = cell ? w * fe.z * rb[1] : 0.0;
+            h += hj;
+        }
+        // ---- k face ---------------------------------------------------------------------------------
+        {
+            const T W = okK ? V.z : T(0);            // (what a face that is not evaluated holds stays out)
+            const V3 fc = ld3(A.kcsi, c), fe = ld3(A.keta, c), fz = ld3(A.kzet, c);
+            const V3 d[3] = {four(uki, ui, shup3(uk), uim),
+                             four(ld3(A.ucat, c + SK + SJ), uj, ld3(A.ucat, c + SK - SJ), ujm), diff(uk, u)};
+            const double nuEff = A.les ? A.nu + 0.5 * (double(n0) + double(nk)) : A.nu;
+            const V3 F = sel(okK, add3v(fb, sc3(-1.0, fbk)));
+            Vec3<T> ukk = uk;
+            if constexpr (QUICK) ukk = ld3(A.ucat, c + 2 * SK);
+            vb.z = opaque_value(okK ? -dot3(F, face_u(ukm, u, uk, ukk, W)) : 0.0);
+            const double nb = adj(std::integral_constant<int, 2>(), okK, F, double(W), d, nuEff, fc, fe, fz, A.kaj[c], cv, G);
+            if (face && okK) A.nueb[2][c] = P(nb);
+            const bool pos = W > T(0);
+            const double wl = QUICK ? (pos ? 0.75 : 0.375) : 0.5, wr = QUICK ? (pos ? 0.375 : 0.75) : 0.5;
+            const V3 ld = sc3(0.25, add3v(up(G[0]), sc3(-1.0, dn(G[0]))));
+            a1 = add3v(a1, add3v(add3v(sc3(wl, cv), sc3(-1.0, G[2])), ld));
+            a2 = add3v(a2, add3v(add3v(sc3(wr, cv), G[2]), ld));
+            if constexpr (QUICK) {
+                a0 = add3v(a0, sc3(pos ? -0.125 : 0.0, cv));
+                a3 = sc3(pos ? 0.0 : -0.125, cv);
+            }
+            tk = sc3(0.25, G[1]);
+            T0 = add3v(T0, tk);
+            hk = cell ? w * fz.z * rb[2] : 0.0;
+            h += hk;
+        }
+        p1 = add3v(p1, T0);
+        JM = add3v(JM, sc3(-1.0, T0));
+        // ---- plane t's jm and theta sums and plane t-1's own and jp sums are complete -----------------
+        if (face) {
+            if (okI && okJ && okK) stp3(A.vbar, c, vb);
+            else {                                     // (the others are the boundary threads' or zero)
+                if (okI) A.vbar[3 * c] = T(vb.x);
+                if (okJ) A.vbar[3 * c + 1] = T(vb.y);
+                if (okK) A.vbar[3 * c + 2] = T(vb.z);
+            }
+            stp3(jm, c, JM);
+            if (A.tbar) { A.tb[c] = h; A.tb[c + n] = hj; }
+        }
+        if (t - 1 >= kb && t - 1 < ke && mine) {
+            const int cm = opaque_index(c0 + (t - 1) * SK);
+            stp3(own, cm, a0);
+            stp3(jp, cm, p0);
+        }
+        a0 = a1; a1 = a2; a2 = a3; a3 = Z;
+        p0 = p1; p1 = p2; p2 = Z;
     }
 }
 
 namespace {
-template <class P>
-__device__ __forceinline__ V3 pk3(const P *pk, long n, int w, int c) {
-    return V3{double(pk[(3 * w + 0) * n + c]), double(pk[(3 * w + 1) * n + c]), double(pk[(3 * w + 2) * n + c])};
+// ucat_bar of point (i, j, k) from the boundary faces' scatter (which only reaches indices up to 2 from
+// either side) and the row sums of k_vjp_march: the row's own, row j-1's jp, row j+1's jm, row j-2's jpp
+template <class T, class P>
+__device__ __forceinline__ V3 row_sums(const VjpArgs<T, P> &A, const Geo &g, int i, int j, int k, int c) {
+    const long n = A.n;
+    const int SJ = g.gxm, jl = g.my - 2;
+    auto get = [&](int q, int p) { return ldp3(A.rows + 3 * q * n, p); };
+    V3 s{0, 0, 0};
+    if (i <= 2 || i >= g.mx - 3 || j <= 2 || j >= g.my - 3 || k <= 2 || k >= g.mz - 3) s = cvt3<double>(ld3(A.ubar, c));
+    if (j >= 1 && j <= jl) s = add3v(s, get(0, c));
+    if (j >= 2 && j <= jl + 1) s = add3v(s, get(1, c - SJ));
+    if (j <= jl - 1) s = add3v(s, get(2, c + SJ));
+    if (A.quick && j >= 3 && j <= jl + 2) s = add3v(s, get(3, c - 2 * SJ));
+    return s;
 }
+// theta_bar of the point: the row's own part and row j-1's j face
+template <class T, class P>
+__device__ __forceinline__ T theta_sum(const VjpArgs<T, P> &A, const Geo &g, int j, int c) {
+    double s = 0.0;
+    if (j >= 1 && j <= g.my - 2) s = A.tb[c];
+    if (j >= 2 && j <= g.my - 1) s += A.tb[A.n + c - g.gxm];
+    return T(s);
+}
+// nu_t_bar of an interior cell is half the nu_eff cotangents of its six faces and of the boundary faces
+// whose ghost nu_t UpdateNutBCs fills from this cell.  Along one axis (x of 1 .. m-2, point stride st) that
+// is hi times the face at the cell's own index and lo times the face `off` points from it: the one below,
+// or the last face for the first cell of a periodic axis, whose face 0 is not evaluated
+struct NuFaces { double hi, lo; int off; };
+template <class A_>
+__device__ __forceinline__ NuFaces nu_faces(const A_ &A, const Geo &g, int q, int x, int st) {
+    const int m = q == 0 ? g.mx : q == 1 ? g.my : g.mz;
+    const int bl = A.bc_nut[2 * q], br = A.bc_nut[2 * q + 1];
+    NuFaces f{x == m - 2 && br == TOSCA_BCNUT_ZEROGRADIENT ? 2.0 : 1.0, 1.0, -st};
+    if (x == 1 && g.per[q] == TOSCA_PERIODIC_NONE) f.lo = bl == TOSCA_BCNUT_ZEROGRADIENT ? 2.0 : 1.0;
+    else if (x == 1) { f.lo = br == TOSCA_BCNUT_PERIODIC ? 1.0 : 0.0; f.off = br == TOSCA_BCNUT_PERIODIC ? (m - 3) * st : -st; }
+    return f;
+}
+// du_center of a cell at index x of an axis, transposed: what its derivative cotangent adds to the cell
+// above, the cell below and the cell itself (one-sided at the first and last cell of a non-periodic axis)
+__device__ __forceinline__ double w_up(bool np, int x, int m) { return np && x == m - 2 ? 0.0 : np && x == 1 ? 1.0 : 0.5; }
+__device__ __forceinline__ double w_dn(bool np, int x, int m) { return np && x == m - 2 ? -1.0 : np && x == 1 ? 0.0 : -0.5; }
+__device__ __forceinline__ double w_own(bool np, int x, int m) { return np && x == m - 2 ? 1.0 : np && x == 1 ? -1.0 : 0.0; }
 }  // namespace
 
 // ------------------------------------------------------------------------------------------------
-// ucat_bar and theta_bar of every owned point (boundary ghosts included): the regular stencils of
-// the interior faces and interior cells, transposed.  Adds to the boundary-face scatter.
+// ucat_bar and theta_bar of every owned point with nu_t = Cs Delta^2 |S| recomputed: the row sums, and the
+// |S| path of the interior cells (nu_t_bar, Cs_bar, the cotangents of the three du_center vectors), which
+// a workgroup of 8 rows marching along k keeps on chip: along i by lane shifts, along j through LDS (one
+// barrier a plane), along k in the accumulators of three planes.  62 x 6 points a workgroup.
+// Bound by latency: 288 bytes a point in FP64, at 3.2 TB/s.  Every load of a cell is issued without a branch
+// (the six faces of nu_t_bar with a condition each took 0.49 ms on the 192 x 192 x 128 hill and 0.86 on the
+// mixed 384 x 256 x 96 box, 0.43 and 0.62 so); loading the row sums ahead of the barrier as well costs
+// 169 registers for 128 and with them half the waves: 0.50 ms.
 // ------------------------------------------------------------------------------------------------
+constexpr int VF_NR = 8, VF_TI = 62, VF_TJ = VF_NR - 2;
 template <class T, class P>
-__global__ void __launch_bounds__(256) k_vjp_gather(VjpArgs<T, P> A, Geo g) {
-    // a workgroup is 64 points along i on 4 consecutive k planes (which read each other's k
-    // neighbours' packets); consecutive workgroups on one XCD take consecutive j rows
-    const int tile = xcd_tile();
-    const int bx = tile % gridDim.x, j = (tile / gridDim.x) % g.my, bk = tile / (gridDim.x * g.my);
-    const int i = bx * 64 + threadIdx.x, k = bk * 4 + threadIdx.y;
-    if (i > g.mx - 1 || k > g.mz - 1) return;
-    const int x[3] = {i, j, k}, m[3] = {g.mx, g.my, g.mz};
-    const int c = g.L(k, j, i);
-    auto Lof = [&](const int *t) { return g.L(t[2], t[1], t[0]); };
-    V3 acc = cvt3<double>(ld3(A.ubar, c));
-    double tb = 0.0;
-    for (int q = 0; q < 3; q++) {
-        const int a = (q == 0) ? 1 : 0, b = (q == 2) ? 1 : 2;          // transverse axes, lower first
-        const P *pk = A.pk[q];
-        // an interior face of direction q at index point t
-        auto faceOK = [&](const int *t) {
-            return t[q] >= 1 && t[q] <= m[q] - 3 && t[a] >= 1 && t[a] <= m[a] - 2 && t[b] >= 1 && t[b] <= m[b] - 2;
+__global__ void __launch_bounds__(64 * VF_NR) k_vjp_finish(VjpArgs<T, P> A, Geo g, int kchunk) {
+    __shared__ double sG[2][3][VF_NR][64];
+    const int lane = threadIdx.x, r = threadIdx.y;
+    const int tile = xcd_tile();                       // j fastest, then i, then the k chunk
+    const int bj = tile % gridDim.y, bi = (tile / gridDim.y) % gridDim.x, bk = tile / (gridDim.x * gridDim.y);
+    const int i = bi * VF_TI + lane - 1, j = bj * VF_TJ + r - 1;
+    const int kb = bk * kchunk, ke = min(kb + kchunk, g.mz);     // points [kb, ke)
+    const bool mine = lane >= 1 && lane <= VF_TI && r >= 1 && r <= VF_TJ && i < g.mx && j < g.my;
+    const bool cellIJ = i >= 1 && i <= g.mx - 2 && j >= 1 && j <= g.my - 2;
+    const bool np0 = g.nonper(0), np1 = g.nonper(1), np2 = g.nonper(2);
+    const double wuI = w_up(np0, i, g.mx), wdI = w_dn(np0, i, g.mx), woI = w_own(np0, i, g.mx), woJ = w_own(np1, j, g.my);
+    const double wuJ = w_up(np1, j - 1, g.my), wdJ = w_dn(np1, j + 1, g.my);     // of the rows below and above
+    const int rm = max(r - 1, 0), rp = min(r + 1, VF_NR - 1);
+    const int SJ = g.gxm, SK = g.gxm * g.gym, jl = g.my - 2;
+    const long n = A.n;
+    const int p0 = g.L(0, min(j, g.my), min(i, g.mx));           // the point in plane 0 (indices from -1)
+    const NuFaces fi = nu_faces(A, g, 0, i, 1), fj = nu_faces(A, g, 1, j, SJ);
+    const bool rOwn = j >= 1 && j <= jl, rJp = j >= 2 && j <= jl + 1, rJm = j <= jl - 1, rJpp = A.quick && j >= 3;
+    const bool edgeIJ = i <= 2 || i >= g.mx - 3 || j <= 2 || j >= g.my - 3;
+    auto get = [&](int q, bool ok, int p) {
+        const V3 v = ldp3(A.rows + 3 * q * n, p);
+        return V3{ok ? v.x : 0.0, ok ? v.y : 0.0, ok ? v.z : 0.0};
+    };
+    V3 c0{0, 0, 0}, c1{0, 0, 0}, c2{0, 0, 0};          // sums of the points of planes k-1, k, k+1
+    Vec3<T> um = ld3(A.ucat, p0 + (kb - 2) * SK), u = ld3(A.ucat, p0 + (kb - 1) * SK);
+    for (int k = kb - 1; k <= ke; k++) {
+        const int buf = k & 1;
+        const bool cell = cellIJ && k >= 1 && k <= g.mz - 2;
+        // every load of the plane without a branch, so that they are in flight together
+        const int c = opaque_index(p0 + k * SK);
+        const NuFaces fk = nu_faces(A, g, 2, k, SK);
+        const double nb = 0.5 * (fi.hi * double(A.nueb[0][c]) + fi.lo * double(A.nueb[0][c + fi.off]) +
+                                 fj.hi * double(A.nueb[1][c]) + fj.lo * double(A.nueb[1][c + fj.off]) +
+                                 fk.hi * double(A.nueb[2][c]) + fk.lo * double(A.nueb[2][c + fk.off]));
+        const V3 cc = ld3(A.csi, c), ee = ld3(A.eta, c), zz = ld3(A.zet, c);
+        const double a = A.aj[c], cs = A.cs[c];
+        const Vec3<T> up = ld3(A.ucat, c + SK);
+        const GradT<T> gr = du_center_v(g, i, j, k, u, ld3(A.ucat, c - 1), ld3(A.ucat, c + 1), ld3(A.ucat, c - SJ),
+                                        ld3(A.ucat, c + SJ), um, up);
+        um = u;
+        u = up;
+        // the strain as the forward computes it (in T), the rest in FP64
+        const CartT<T> dT = du_dxyz(cvt3<T>(cc), cvt3<T>(ee), cvt3<T>(zz), T(a), gr);
+        const double S = double(strain_mag(dT));
+        const double filter = cube_root(1. / a), d2 = filter * filter;
+        if (cell && mine && k >= kb && k < ke) A.csbar[c] = nb * d2 * S;
+        // d|S| / dD_mn = 2 S_mn / |S|, S = sym(D); |S| is not differentiable at 0: subgradient 0
+        const bool on = cell && S != 0.0 && nb != 0.0;
+        const double sb = nb * cs * d2 * 2.0 / S;
+        const double Sxx = dT.du_dx, Sxy = 0.5 * (double(dT.du_dy) + double(dT.dv_dx)), Sxz = 0.5 * (double(dT.du_dz) + double(dT.dw_dx));
+        const double Syy = dT.dv_dy, Syz = 0.5 * (double(dT.dv_dz) + double(dT.dw_dy)), Szz = dT.dw_dz;
+        const V3 Du{sb * Sxx, sb * Sxy, sb * Sxz}, Dv{sb * Sxy, sb * Syy, sb * Syz}, Dw{sb * Sxz, sb * Syz, sb * Szz};
+        // D_m. = aj (d_c u_m csi + d_e u_m eta + d_z u_m zet)  ->  d_X u_m bar = aj (Dbar_m . M_X)
+        auto bar = [&](V3 M) {
+            const V3 v{a * dot3(Du, M), a * dot3(Dv, M), a * dot3(Dw, M)};
+            return V3{on ? v.x : 0.0, on ? v.y : 0.0, on ? v.z : 0.0};
         };
-        int t[3];
-        // normal derivative and convective interpolation: x is the left cell of face x, the right
-        // cell of face x - q; QUICK also reaches x from faces x + q (V > 0) and x - 2q (V <= 0)
-        for (int s = -2; s <= 1; s++) {
-            t[0] = i; t[1] = j; t[2] = k;
-            t[q] = x[q] + s;
-            if (!faceOK(t)) continue;
-            const int fc = Lof(t);
-            const V3 cv = pk3(pk, A.n, 0, fc);
-            if (s == 0 || s == -1) {
-                const V3 gn = pk3(pk, A.n, 1, fc);
-                acc = add3v(acc, sc3(s == 0 ? -1.0 : 1.0, gn));
-            }
-            double w;
-            if (!A.quick) w = (s == 0 || s == -1) ? 0.5 : 0.0;
-            else {
-                const bool pos = A.ucont[3 * fc + q] > T(0);
-                if (s == 0) w = pos ? 0.75 : 0.375;
-                else if (s == -1) w = pos ? 0.375 : 0.75;
-                else if (s == 1) w = pos ? -0.125 : 0.0;
-                else w = pos ? 0.0 : -0.125;
-            }
-            if (w != 0.0) acc = add3v(acc, sc3(w, cv));
+        const V3 gc = bar(cc), ge = bar(ee), gz = bar(zz);
+        sG[buf][0][r][lane] = ge.x; sG[buf][1][r][lane] = ge.y; sG[buf][2][r][lane] = ge.z;
+        // own cell, then the cells along i
+        const double woK = w_own(np2, k, g.mz);
+        c1 = add3v(c1, add3v(sc3(woI, gc), add3v(sc3(woJ, ge), sc3(woK, gz))));
+        c1 = add3v(c1, add3v(shup3(sc3(wuI, gc)), shdn3(sc3(wdI, gc))));
+        c2 = add3v(c2, sc3(w_up(np2, k, g.mz), gz));
+        c0 = add3v(c0, sc3(w_dn(np2, k, g.mz), gz));
+        __syncthreads();                               // the other buffer is rewritten behind the next one
+        c1 = add3v(c1, V3{wuJ * sG[buf][0][rm][lane] + wdJ * sG[buf][0][rp][lane],
+                          wuJ * sG[buf][1][rm][lane] + wdJ * sG[buf][1][rp][lane],
+                          wuJ * sG[buf][2][rm][lane] + wdJ * sG[buf][2][rp][lane]});
+        if (mine && k - 1 >= kb && k - 1 < ke) {       // the points of plane k-1 are complete
+            const int cm = opaque_index(p0 + (k - 1) * SK);
+            stp3(A.ubar, cm, add3v(row_sums(A, g, i, j, k - 1, cm), c0));
+            if (A.tbar) A.tbar[cm] = theta_sum(A, g, j, cm);
         }
-        // transverse four-point averages: faces x - e and x - e - q add, x + e and x + e - q subtract
-        for (int e = 0; e < 2; e++) {
-            const int ax = e == 0 ? a : b;
-            for (int sgn = -1; sgn <= 1; sgn += 2) {
-                for (int sq = 0; sq <= 1; sq++) {
-                    t[0] = i; t[1] = j; t[2] = k;
-                    t[ax] = x[ax] + sgn;
-                    t[q] = x[q] - sq;
-                    if (!faceOK(t)) continue;
-                    const V3 gt = pk3(pk, A.n, 2 + e, Lof(t));
-                    acc = add3v(acc, sc3(-0.25 * sgn, gt));
-                }
-            }
-        }
-        // |S| path: du_center of the interior cells x - q, x, x + q along q
-        if (A.les && !A.nut_in) {
-            const bool np = g.per[q] == TOSCA_PERIODIC_NONE;
-            auto cellOK = [&](const int *t) {
-                return t[0] >= 1 && t[0] <= m[0] - 2 && t[1] >= 1 && t[1] <= m[1] - 2 && t[2] >= 1 && t[2] <= m[2] - 2;
-            };
-            for (int s = -1; s <= 1; s++) {
-                t[0] = i; t[1] = j; t[2] = k;
-                t[q] = x[q] + s;
-                if (!cellOK(t)) continue;
-                const int cq = t[q];
-                double w = 0.0;
-                if (s == 1) w = (np && cq == m[q] - 2) ? -1.0 : (np && cq == 1) ? 0.0 : -0.5;
-                else if (s == -1) w = (np && cq == m[q] - 2) ? 0.0 : (np && cq == 1) ? 1.0 : 0.5;
-                else w = (np && cq == m[q] - 2) ? 1.0 : (np && cq == 1) ? -1.0 : 0.0;
-                if (w != 0.0) acc = add3v(acc, sc3(w, pk3(A.spk, A.n, q, Lof(t))));
-            }
-        }
-        // buoyancy: the + face q of this cell and of the cell below along q
-        if (!A.tbar) continue;
-        for (int s = -1; s <= 0; s++) {
-            t[0] = i; t[1] = j; t[2] = k;
-            t[q] = x[q] + s;
-            if (t[0] < 1 || t[0] > m[0] - 2 || t[1] < 1 || t[1] > m[1] - 2 || t[2] < 1 || t[2] > m[2] - 2) continue;
-            const int cb = Lof(t);
-            const double *face = (q == 0) ? A.icsi : (q == 1) ? A.jeta : A.kzet;
-            tb += -A.bscale * (-9.81 * face[3 * cb + 2]) * 0.5 / A.tRef * A.rbar[3 * g.G(t[2], t[1], t[0]) + q];
-        }
+        c0 = c1; c1 = c2; c2 = V3{0, 0, 0};
     }
-    stp3(A.ubar, c, acc);
-    if (A.tbar) A.tbar[c] = T(tb);
 }
 
 // ------------------------------------------------------------------------------------------------
-// nu_t as an input array: its cotangent at every owned point, accumulated (+=).  The face of
-// direction q at index point c averages nu_t of cells c and c + e_q, so point c collects half the
-// nu_eff cotangent of faces c and c - e_q (zero where a face is not evaluated).
+// The same without the |S| path (no LES, or nu_t an input array): one thread per owned point.  With nu_t
+// an input its cotangent is accumulated (+=): the face of direction q at index point c averages nu_t of
+// cells c and c + e_q, so point c collects half the nu_eff cotangent of faces c and c - e_q (zero where a
+// face is not evaluated).
 // ------------------------------------------------------------------------------------------------
 template <class T, class P>
-__global__ void __launch_bounds__(256) k_vjp_nutbar(VjpArgs<T, P> A, Geo g) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y, k = blockIdx.z;
-    if (i > g.mx - 1) return;
+__global__ void __launch_bounds__(256) k_vjp_sum(VjpArgs<T, P> A, Geo g) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y * blockDim.y + threadIdx.y, k = blockIdx.z;
+    if (i > g.mx - 1 || j > g.my - 1) return;
     const int c = g.L(k, j, i);
-    const double s = double(A.nueb[0][c]) + double(A.nueb[0][g.L(k, j, i - 1)]) + double(A.nueb[1][c]) +
-                     double(A.nueb[1][g.L(k, j - 1, i)]) + double(A.nueb[2][c]) + double(A.nueb[2][g.L(k - 1, j, i)]);
-    A.nutbar_acc[c] += 0.5 * s;
+    stp3(A.ubar, c, row_sums(A, g, i, j, k, c));
+    if (A.tbar) A.tbar[c] = theta_sum(A, g, j, c);
+    if (A.les && A.nutbar_acc) {
+        const double s = double(A.nueb[0][c]) + double(A.nueb[0][g.L(k, j, i - 1)]) + double(A.nueb[1][c]) +
+                         double(A.nueb[1][g.L(k, j - 1, i)]) + double(A.nueb[2][c]) + double(A.nueb[2][g.L(k - 1, j, i)]);
+        A.nutbar_acc[c] += 0.5 * s;
+    }
 }
 
 // The transposed stages on the stream.  cs != nullptr: nu_t = UpdateNut(ucat, cs) is recomputed
 // and differentiated (Cs_bar, |S| path); nut_in != nullptr: nu_t is an input and its cotangent is
-// added to nut_bar.  theta_bar == nullptr: no Buoyancy term.  ws: n values of T for nu_t, then
-// 51 n values of P for the intermediates (52 n doubles cover both forms).
+// added to nut_bar.  theta_bar == nullptr: no Buoyancy term.  ws (vjp_ws_doubles): n values of T for
+// nu_t, 2 n doubles for tb, then 18 n values of P for fpbar, nueb and the row sums.
 template <class T, class P>
 void vjp_rhs_impl(const Geo &g, const tosca_mesh *mesh, const tosca_params *p, const T *ucont, const T *ucat,
                   const double *cs, const T *nut_in, const double *rbar, double scale, double buoy_scale, T *ucont_bar,
                   T *ucat_bar, T *theta_bar, double *cs_bar, double *nut_bar, double *ws, hipStream_t s) {
     const long n = g.nloc();
     T *nut = reinterpret_cast<T *>(ws);
-    P *base = reinterpret_cast<P *>(ws + n);
-    P *fpbar = base, *nueb = base + 3 * n, *spk = base + 6 * n, *pk = base + 15 * n;   // 51 n values of P
-    const dim3 zb(256), zg(2048);
-    TOSCA_LAUNCH("k_vjp_zero", k_vjp_zero<T>, zg, zb, 0, s, ucont_bar, 3 * n);
-    TOSCA_LAUNCH("k_vjp_zero", k_vjp_zero<T>, zg, zb, 0, s, ucat_bar, 3 * n);
-    if (theta_bar) TOSCA_LAUNCH("k_vjp_zero", k_vjp_zero<T>, zg, zb, 0, s, theta_bar, n);
-    if (cs_bar) launch_fill(cs_bar, n, 0.0, s);
-    TOSCA_LAUNCH("k_vjp_zero", k_vjp_zero<P>, zg, zb, 0, s, nueb, 3 * n);
+    P *base = reinterpret_cast<P *>(ws + 3 * n);
+    P *fpbar = base, *nueb = base + 3 * n;
     const bool les = p->les_active != 0;
     const bool renut = les && !nut_in;      // nu_t recomputed as the forward step does (k_vjp_pre)
+    // what no later kernel writes: ucont_bar, nueb and cs_bar outside the interior cells (k_vjp_march writes
+    // every face of theirs), theta_bar outside the owned points; and the layers of
+    // ucat_bar the boundary faces scatter into
+    ZeroShells Z{};
+    auto zero = [&](void *p, int words, int w) { if (p) { Z.p[Z.n] = static_cast<unsigned *>(p); Z.words[Z.n] = words; Z.w[Z.n++] = w; } };
+    const int wT = sizeof(T) / 4, wP = sizeof(P) / 4;
+    zero(ucont_bar, 3 * wT, GW + 1);
+    zero(ucat_bar, 3 * wT, GW + 3);
+    zero(theta_bar, wT, GW);
+    zero(cs_bar, 2, renut ? GW + 1 : g.gzm);           // (without the |S| path, all of it)
+    for (int q = 0; q < 3; q++) zero(nueb + q * n, wP, GW + 1);
+    TOSCA_LAUNCH("k_vjp_zero", k_vjp_zero_shells, dim3(256, 6, Z.n), dim3(256), 0, s, Z, g);
     VjpArgs<T, P> A;
     A.ucont = ucont; A.ucat = ucat; A.theta = nullptr; A.cs = cs; A.rbar = rbar;
     A.nut = les ? (nut_in ? nut_in : nut) : ucat;
@@ -553,8 +759,9 @@ void vjp_rhs_impl(const Geo &g, const tosca_mesh *mesh, const tosca_params *p, c
     A.tauI = p->tau_wall_i; A.tauJ = p->tau_wall_j;
     A.fpbar = fpbar; A.nutbar_acc = nut_bar;
     A.vbar = ucont_bar; A.ubar = ucat_bar; A.tbar = theta_bar; A.csbar = cs_bar;
-    for (int q = 0; q < 3; q++) { A.pk[q] = pk + 12 * q * n; A.nueb[q] = nueb + q * n; }
-    A.spk = spk;
+    for (int q = 0; q < 3; q++) A.nueb[q] = nueb + q * n;
+    A.rows = base + 6 * n;
+    A.tb = ws + n;
     A.n = n;
     A.scale = scale; A.bscale = buoy_scale; A.tRef = p->t_ref; A.nu = p->nu;
     A.quick = p->div_scheme == TOSCA_DIV_QUICK;
@@ -570,15 +777,25 @@ void vjp_rhs_impl(const Geo &g, const tosca_mesh *mesh, const tosca_params *p, c
     } else {
         TOSCA_LAUNCH(f32 ? "k_vjp_fp_f32" : "k_vjp_fp", (k_vjp_fp<T, P>), cg, cb, 0, s, A, g);
     }
-    // faces: x along i (0 .. mx-2 for i faces, 1 .. mx-2 otherwise), y / z the other two axes
-    TOSCA_LAUNCH(f32 ? "k_vjp_faces_f32" : "k_vjp_faces", (k_vjp_faces<T, P>), dim3((g.mx - 1 + 255) / 256, g.my - 1, g.mz - 1),
-                 dim3(256), 0, s, A, g);
-    if (les && !nut_in) TOSCA_LAUNCH(f32 ? "k_vjp_nut_f32" : "k_vjp_nut", (k_vjp_nut<T, P>), cg, cb, 0, s, A, g);
-    if (les && nut_in)
-        TOSCA_LAUNCH("k_vjp_nutbar", (k_vjp_nutbar<T, P>), dim3((g.mx + 255) / 256, g.my, g.mz), dim3(256), 0, s, A, g);
-    TOSCA_LAUNCH(f32 ? "k_vjp_gather_f32" : "k_vjp_gather", (k_vjp_gather<T, P>), dim3((g.mx + 63) / 64, (g.mz + 3) / 4, g.my),
-                 dim3(64, 4), 0, s, A, g);
+    const int ti = (g.mx + 59) / 60, tj = (g.my - 2 + 3) / 4;
+    const int kc = plane_chunk(g.mz, ti * tj, 2 * NUM_CU, 3, 2000.0);
+    const int nmax = max(g.my * g.mz, max(g.mx * g.mz, g.mx * g.my));
+    const int nbnd = (6 * nmax + 2047) / 2048 * 8;     // workgroups of 256 boundary faces, a multiple of the XCDs
+    const dim3 mg(nbnd + ti * tj * ((g.mz + kc - 1) / kc));
+    if (A.quick) TOSCA_LAUNCH(f32 ? "k_vjp_march_f32" : "k_vjp_march", (k_vjp_march<T, P, true>), mg, dim3(64, 4), 0, s, A, g, kc, ti, tj, nbnd, nmax);
+    else TOSCA_LAUNCH(f32 ? "k_vjp_march_f32" : "k_vjp_march", (k_vjp_march<T, P, false>), mg, dim3(64, 4), 0, s, A, g, kc, ti, tj, nbnd, nmax);
+    if (renut) {
+        const int fi = (g.mx + VF_TI - 1) / VF_TI, fj = (g.my + VF_TJ - 1) / VF_TJ;
+        const int fc = plane_chunk(g.mz, fi * fj, 2 * NUM_CU, 2, 500.0);
+        TOSCA_LAUNCH(f32 ? "k_vjp_finish_f32" : "k_vjp_finish", (k_vjp_finish<T, P>), dim3(fi, fj, (g.mz + fc - 1) / fc),
+                     dim3(64, VF_NR), 0, s, A, g, fc);
+    } else {
+        TOSCA_LAUNCH(f32 ? "k_vjp_sum_f32" : "k_vjp_sum", (k_vjp_sum<T, P>), dim3((g.mx + 63) / 64, (g.my + 3) / 4, g.mz),
+                     dim3(64, 4), 0, s, A, g);
+    }
 }
+
+size_t vjp_ws_doubles(const Geo &g) { return 21 * (size_t)g.nloc(); }
 
 void vjp_rhs(const Geo &g, const tosca_mesh *mesh, const tosca_params *p, const double *ucont, const double *ucat,
              const double *theta, const double *cs, const double *rbar, double scale, double buoy_scale,
