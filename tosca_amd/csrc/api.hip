@@ -262,9 +262,9 @@ size_t ws_need(const tosca_ctx *c, const tosca_params *p) {
     // reference-structured path: FormU's 6 face-flux vectors + fp (21 local fields), UpdateCs's
     // strain rows, LM/MM/QN/NN and the DPASD plane partials
     if (c->ref_path) return 22 * n + (size_t)c->geo.my * 16 * 4 + 64;
-    // fused path: LM, MM, |S| then FormU's boundary-face and seam buffers; FormT's two face-flux
-    // vectors; the DPASD filter sums when that model runs
-    size_t need = std::max(3 * n + tosca::formu_ws_doubles(c->geo) + 64, 6 * n + 64);
+    // fused path: LM, MM, |S| then FormU's boundary-face and seam buffers; the DPASD filter sums when
+    // that model runs
+    size_t need = 3 * n + tosca::formu_ws_doubles(c->geo) + 64;
     if (p && p->les_active && p->les_model == TOSCA_LES_DPASD) need = std::max(need, tosca::dpasd_ws_doubles(c->geo));
     return need;
 }
@@ -1289,8 +1289,7 @@ int tosca_formt(tosca_ctx *c, const tosca_mesh *m, const tosca_params *p, const 
             (rc = check_dev(c, tp->q_wall_j, 3 * (size_t)g.mz * g.mx * sizeof(double), "q_wall_j")))
             return rc;
     }
-    if ((rc = ensure_ws(c, ws_need(c, p)))) return rc;
-    tosca::ref_formt(g, m, p, tp, ucont, theta, nut, kt, rhs, scale, form_mode, c->ws, c->stream);
+    tosca::formt(g, m, p, tp, ucont, theta, nut, kt, rhs, scale, form_mode, c->stream);
     return launched(c, "FormT");
 }
 

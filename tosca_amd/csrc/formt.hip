@@ -2,17 +2,13 @@
 // potential-temperature equation and their cell budgets, on gfx950.  Compiled with FP contraction
 // off: every face flux is evaluated in the reference's expression order.
 //
-//   k_formt_faces   the fused i/j/k face loop (teqn_solvers.c:117-481): WENO3 upwinded advective
-//                   flux and the diffusive flux with the effective diffusivity of the LES closure
-//                   (nu/Pr, the subgrid diffusivity k_t, or nu_t over the stability-corrected
-//                   turbulent Prandtl number) and the wall heat flux of thetaWallFunction patches
-//   (ghosts)        DMLocalToLocal and resetFacePeriodicFluxesVector on both flux arrays (:487-503)
-//   k_formt_cells   the flux budgets of the interior cells times the cell Jacobian (:511-537)
-//
-// Flux arrays are two local vector fields in the context workspace; the faces kernel covers the
-// whole ghosted range and writes zero where the reference leaves its VecSet(0) value, so no
-// separate clear is needed.
-#include "kernels.h"
+//   k_formt   the fused i/j/k face loop (teqn_solvers.c:117-481): WENO3 upwinded advective flux and
+//             the diffusive flux with the effective diffusivity of the LES closure (nu/Pr, the subgrid
+//             diffusivity k_t, or nu_t over the stability-corrected turbulent Prandtl number) and the
+//             wall heat flux of thetaWallFunction patches; face 0 of a periodic axis taken as face m-2
+//             (resetFacePeriodicFluxesVector, :487-503); the flux budgets of the interior cells times
+//             the cell Jacobian (:511-537).  The fluxes never reach memory.
+#include "fused.h"
 
 namespace tosca {
 
@@ -23,69 +19,20 @@ struct FormTArgs {
     const double *icsi, *ieta, *izet, *jcsi, *jeta, *jzet, *kcsi, *keta, *kzet;
     const double *iaj, *jaj, *kaj;
     const double *qI, *qJ;       // wall heat flux [3][mz][my] (i patches), [3][mz][mx] (j patches)
-    double *div, *visc;          // local vector fields
-    double nu, pr, tref;
-    int les, ktm, wall[4];
+    const double *aj;
+    double *rhs;
+    double nu, pr, tref, scale;
+    int wall[4], mode;
 };
 
-// Compute_dscalar_i / _j / _k (src/include/inline.h:3210-3342) with no IBM or overset cells: the
-// difference across the face and the two four-point transverse averages, which become two-point
-// one-sided averages on the face rows next to a non-periodic boundary edge.
-__device__ __forceinline__ void dscalar_i(const Geo &g, const double *K, int i, int j, int k, double &dc, double &de,
-                                          double &dz) {
-    const bool iN = g.nonper(0), jN = g.nonper(1), kN = g.nonper(2);
-    const bool ib = (i == 0 || i == g.mx - 2);
-    dc = K[g.L(k, j, i + 1)] - K[g.L(k, j, i)];
-    if (j == g.my - 2 && ib && (jN || iN))
-        de = (K[g.L(k, j, i + 1)] + K[g.L(k, j, i)] - K[g.L(k, j - 1, i + 1)] - K[g.L(k, j - 1, i)]) * 0.5;
-    else if (j == 1 && ib && (jN || iN))
-        de = (K[g.L(k, j + 1, i + 1)] + K[g.L(k, j + 1, i)] - K[g.L(k, j, i + 1)] - K[g.L(k, j, i)]) * 0.5;
-    else
-        de = (K[g.L(k, j + 1, i + 1)] + K[g.L(k, j + 1, i)] - K[g.L(k, j - 1, i + 1)] - K[g.L(k, j - 1, i)]) * 0.25;
-    if (k == g.mz - 2 && ib && (kN || iN))
-        dz = (K[g.L(k, j, i + 1)] + K[g.L(k, j, i)] - K[g.L(k - 1, j, i + 1)] - K[g.L(k - 1, j, i)]) * 0.5;
-    else if (k == 1 && ib && (kN || iN))
-        dz = (K[g.L(k + 1, j, i + 1)] + K[g.L(k + 1, j, i)] - K[g.L(k, j, i + 1)] - K[g.L(k, j, i)]) * 0.5;
-    else
-        dz = (K[g.L(k + 1, j, i + 1)] + K[g.L(k + 1, j, i)] - K[g.L(k - 1, j, i + 1)] - K[g.L(k - 1, j, i)]) * 0.25;
-}
-
-__device__ __forceinline__ void dscalar_j(const Geo &g, const double *K, int i, int j, int k, double &dc, double &de,
-                                          double &dz) {
-    const bool iN = g.nonper(0), jN = g.nonper(1), kN = g.nonper(2);
-    const bool jb = (j == 0 || j == g.my - 2);
-    if (i == g.mx - 2 && jb && (iN || jN))
-        dc = (K[g.L(k, j + 1, i)] + K[g.L(k, j, i)] - K[g.L(k, j + 1, i - 1)] - K[g.L(k, j, i - 1)]) * 0.5;
-    else if (i == 1 && jb && (iN || jN))
-        dc = (K[g.L(k, j + 1, i + 1)] + K[g.L(k, j, i + 1)] - K[g.L(k, j + 1, i)] - K[g.L(k, j, i)]) * 0.5;
-    else
-        dc = (K[g.L(k, j + 1, i + 1)] + K[g.L(k, j, i + 1)] - K[g.L(k, j + 1, i - 1)] - K[g.L(k, j, i - 1)]) * 0.25;
-    de = K[g.L(k, j + 1, i)] - K[g.L(k, j, i)];
-    if (k == g.mz - 2 && jb && (kN || jN))
-        dz = (K[g.L(k, j + 1, i)] + K[g.L(k, j, i)] - K[g.L(k - 1, j + 1, i)] - K[g.L(k - 1, j, i)]) * 0.5;
-    else if (k == 1 && jb && (kN || jN))
-        dz = (K[g.L(k + 1, j + 1, i)] + K[g.L(k + 1, j, i)] - K[g.L(k, j + 1, i)] - K[g.L(k, j, i)]) * 0.5;
-    else
-        dz = (K[g.L(k + 1, j + 1, i)] + K[g.L(k + 1, j, i)] - K[g.L(k - 1, j + 1, i)] - K[g.L(k - 1, j, i)]) * 0.25;
-}
-
-__device__ __forceinline__ void dscalar_k(const Geo &g, const double *K, int i, int j, int k, double &dc, double &de,
-                                          double &dz) {
-    const bool iN = g.nonper(0), jN = g.nonper(1), kN = g.nonper(2);
-    const bool kb = (k == 0 || k == g.mz - 2);
-    if (i == g.mx - 2 && kb && (iN || kN))
-        dc = (K[g.L(k + 1, j, i)] + K[g.L(k, j, i)] - K[g.L(k + 1, j, i - 1)] - K[g.L(k, j, i - 1)]) * 0.5;
-    else if (i == 1 && kb && (iN || kN))
-        dc = (K[g.L(k + 1, j, i + 1)] + K[g.L(k, j, i + 1)] - K[g.L(k + 1, j, i)] - K[g.L(k, j, i)]) * 0.5;
-    else
-        dc = (K[g.L(k + 1, j, i + 1)] + K[g.L(k, j, i + 1)] - K[g.L(k + 1, j, i - 1)] - K[g.L(k, j, i - 1)]) * 0.25;
-    if (j == g.my - 2 && kb && (jN || kN))
-        de = (K[g.L(k + 1, j, i)] + K[g.L(k, j, i)] - K[g.L(k + 1, j - 1, i)] - K[g.L(k, j - 1, i)]) * 0.5;
-    else if (j == 1 && kb && (jN || kN))
-        de = (K[g.L(k + 1, j + 1, i)] + K[g.L(k, j + 1, i)] - K[g.L(k + 1, j, i)] - K[g.L(k, j, i)]) * 0.5;
-    else
-        de = (K[g.L(k + 1, j + 1, i)] + K[g.L(k, j + 1, i)] - K[g.L(k + 1, j - 1, i)] - K[g.L(k, j - 1, i)]) * 0.25;
-    dz = K[g.L(k + 1, j, i)] - K[g.L(k, j, i)];
+// Compute_dscalar_i / _j / _k (src/include/inline.h:3210-3342) with no IBM or overset cells, across the
+// face and its two transverse axes: four-point transverse averages, which become two-point one-sided
+// averages on the face rows next to a non-periodic boundary edge.  Along a transverse axis (index x of
+// 1 .. m-2, point stride st): the offsets of the two rows and the weight.
+struct Across { int hi, lo; double w; };
+__device__ __forceinline__ Across across(bool edge, int x, int m, int st) {
+    const bool top = edge && x == m - 2, bot = edge && x == 1 && !top;
+    return Across{top ? 0 : st, bot ? 0 : -st, top || bot ? 0.5 : 0.25};
 }
 
 // getFace2Cell4Stencil{Csi,Eta,Zet} (src/include/inline.h:2190-2330): the outer cells of the
@@ -126,14 +73,16 @@ __device__ __forceinline__ double weno3(double f0, double f1, double f2, double 
 // carry one, else nu_t over the turbulent Prandtl number 1 / (1 + 2 l / delta), with the
 // stability length l = min(delta, 7.6 nu_t / delta sqrt(T_ref / |g . grad T|)) in stable
 // stratification (g . grad T < 0) and l = delta otherwise
-__device__ __forceinline__ double kappa_eff(const FormTArgs &A, long c, long cn, double ajc, double dtde) {
-    if (!A.les) return A.nu / A.pr;
+enum { KAP_NONE, KAP_KT, KAP_NUT };      // no LES, a model that carries k_t, nu_t over Pr_t
+template <int KAP>
+__device__ __forceinline__ double kappa_eff(const FormTArgs &A, int c, int cn, double ajc, double dtde) {
+    if constexpr (KAP == KAP_NONE) return A.nu / A.pr;
     const double nu = 0.0;
-    const double nut = 0.5 * (A.nut[c] + A.nut[cn]);
-    if (A.ktm) {
+    if constexpr (KAP == KAP_KT) {
         const double diff = 0.5 * (A.kt[c] + A.kt[cn]);
         return (nu / A.pr) + diff;
     }
+    const double nut = 0.5 * (A.nut[c] + A.nut[cn]);
     const double gradTdotG = dtde * (-9.81);
     const double delta = pow(1. / ajc, 1. / 3.);
     double l;
@@ -147,106 +96,98 @@ __device__ __forceinline__ double kappa_eff(const FormTArgs &A, long c, long cn,
 }
 
 // The advective (d) and diffusive (v) flux of one face, as the reference's face loop evaluates it
-// (teqn_solvers.c:127-246 / 250-370 / 374-478).  Face (k, j, i) of direction DIR lies between
-// cell (k, j, i) and its + neighbour along DIR.
-__device__ __forceinline__ void flux_i(const FormTArgs &A, const Geo &g, int i, int j, int k, double &d, double &v) {
+// (teqn_solvers.c:127-246 / 250-370 / 374-478).  Face (i, j, k) of direction DIR lies between cell
+// (i, j, k), local index c, and its + neighbour along DIR.
+template <int DIR, int KAP>
+__device__ __forceinline__ void face_flux(const FormTArgs &A, const Geo &g, int i, int j, int k, int c, double &d, double &v) {
     const double *T = A.t;
-    const long c = g.L(k, j, i);
-    const double ajc = A.iaj[c];
-    const V3 cs = ld3(A.icsi, c), et = ld3(A.ieta, c), ze = ld3(A.izet, c);
-    const double g11 = cs.x * cs.x + cs.y * cs.y + cs.z * cs.z;
-    const double g21 = et.x * cs.x + et.y * cs.y + et.z * cs.z;
-    const double g31 = ze.x * cs.x + ze.y * cs.y + ze.z * cs.z;
-    double dtdc, dtde, dtdz;
-    dscalar_i(g, T, i, j, k, dtdc, dtde, dtdz);
-    int iL, iR;
-    face_stencil(g.per[0], i, g.mx, iL, iR);
-    const double u = A.ucont[3 * c];
-    d = -u * weno3(T[g.L(k, j, iL)], T[c], T[g.L(k, j, i + 1)], T[g.L(k, j, iR)], u);
-    double kap = kappa_eff(A, c, g.L(k, j, i + 1), ajc, dtde);
-    v = 0.0;
-    if (A.les && ((A.wall[0] && i == 0) || (A.wall[1] && i == g.mx - 2))) {
-        const double signQ = (i == 0) ? -1.0 : 1.0;
-        const long pl = (long)g.mz * g.my, o = (long)k * g.my + j;
-        v = signQ * (A.qI[o] * cs.x + A.qI[pl + o] * cs.y + A.qI[2 * pl + o] * cs.z);
-        kap = 0.0;
+    const int x[3] = {i, j, k}, m[3] = {g.mx, g.my, g.mz}, st[3] = {1, g.gxm, g.gxm * g.gym};
+    const int f = x[DIR], sd = st[DIR];
+    const double ajc = (DIR == 0 ? A.iaj : DIR == 1 ? A.jaj : A.kaj)[c];
+    const V3 cs = ld3(DIR == 0 ? A.icsi : DIR == 1 ? A.jcsi : A.kcsi, c), et = ld3(DIR == 0 ? A.ieta : DIR == 1 ? A.jeta : A.keta, c),
+             ze = ld3(DIR == 0 ? A.izet : DIR == 1 ? A.jzet : A.kzet, c);
+    const double T0 = T[c], T1 = T[c + sd];
+    double dt[3];
+    const bool edge = f == 0 || f == m[DIR] - 2;
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        if (q == DIR) { dt[q] = T1 - T0; continue; }
+        const Across a = across(edge && (g.nonper(q) || g.nonper(DIR)), x[q], m[q], st[q]);
+        dt[q] = (T[c + sd + a.hi] + T[c + a.hi] - T[c + sd + a.lo] - T[c + a.lo]) * a.w;
     }
-    v += (g11 * dtdc + g21 * dtde + g31 * dtdz) * ajc * kap;
-}
-
-__device__ __forceinline__ void flux_j(const FormTArgs &A, const Geo &g, int i, int j, int k, double &d, double &v) {
-    const double *T = A.t;
-    const long c = g.L(k, j, i);
-    const double ajc = A.jaj[c];
-    const V3 cs = ld3(A.jcsi, c), et = ld3(A.jeta, c), ze = ld3(A.jzet, c);
-    const double g11 = cs.x * et.x + cs.y * et.y + cs.z * et.z;
-    const double g21 = et.x * et.x + et.y * et.y + et.z * et.z;
-    const double g31 = ze.x * et.x + ze.y * et.y + ze.z * et.z;
-    double dtdc, dtde, dtdz;
-    dscalar_j(g, T, i, j, k, dtdc, dtde, dtdz);
-    int jL, jR;
-    face_stencil(g.per[1], j, g.my, jL, jR);
-    const double u = A.ucont[3 * c + 1];
-    d = -u * weno3(T[g.L(k, jL, i)], T[c], T[g.L(k, j + 1, i)], T[g.L(k, jR, i)], u);
-    double kap = kappa_eff(A, c, g.L(k, j + 1, i), ajc, dtde);
+    int L, R;
+    face_stencil(g.per[DIR], f, m[DIR], L, R);
+    const double u = A.ucont[3 * c + DIR];
+    d = -u * weno3(T[c + (L - f) * sd], T0, T1, T[c + (R - f) * sd], u);
+    double kap = kappa_eff<KAP>(A, c, c + sd, ajc, dt[1]);
+    const V3 n = DIR == 0 ? cs : DIR == 1 ? et : ze;
+    const double g11 = cs.x * n.x + cs.y * n.y + cs.z * n.z;
+    const double g21 = et.x * n.x + et.y * n.y + et.z * n.z;
+    const double g31 = ze.x * n.x + ze.y * n.y + ze.z * n.z;
     v = 0.0;
-    if (A.les && ((A.wall[2] && j == 0) || (A.wall[3] && j == g.my - 2))) {
-        const double signQ = (j == 0) ? -1.0 : 1.0;
-        const long pl = (long)g.mz * g.mx, o = (long)k * g.mx + i;
-        v = signQ * (A.qJ[o] * et.x + A.qJ[pl + o] * et.y + A.qJ[2 * pl + o] * et.z);
-        kap = 0.0;
+    if (DIR < 2) {
+        if (KAP != KAP_NONE && ((A.wall[DIR < 2 ? 2 * DIR : 0] && f == 0) || (A.wall[DIR < 2 ? 2 * DIR + 1 : 0] && f == m[DIR] - 2))) {
+            const double signQ = (f == 0) ? -1.0 : 1.0;
+            const double *q = DIR == 0 ? A.qI : A.qJ;
+            const int n1 = DIR == 0 ? g.my : g.mx, pl = g.mz * n1, o = k * n1 + (DIR == 0 ? j : i);
+            v = signQ * (q[o] * n.x + q[pl + o] * n.y + q[2 * pl + o] * n.z);
+            kap = 0.0;
+        }
     }
-    v += (g11 * dtdc + g21 * dtde + g31 * dtdz) * ajc * kap;
+    v += (g11 * dt[0] + g21 * dt[1] + g31 * dt[2]) * ajc * kap;
 }
 
-__device__ __forceinline__ void flux_k(const FormTArgs &A, const Geo &g, int i, int j, int k, double &d, double &v) {
-    const double *T = A.t;
-    const long c = g.L(k, j, i);
-    const double ajc = A.kaj[c];
-    const V3 cs = ld3(A.kcsi, c), et = ld3(A.keta, c), ze = ld3(A.kzet, c);
-    const double g11 = cs.x * ze.x + cs.y * ze.y + cs.z * ze.z;
-    const double g21 = et.x * ze.x + et.y * ze.y + et.z * ze.z;
-    const double g31 = ze.x * ze.x + ze.y * ze.y + ze.z * ze.z;
-    double dtdc, dtde, dtdz;
-    dscalar_k(g, T, i, j, k, dtdc, dtde, dtdz);
-    int kL, kR;
-    face_stencil(g.per[2], k, g.mz, kL, kR);
-    const double u = A.ucont[3 * c + 2];
-    d = -u * weno3(T[g.L(kL, j, i)], T[c], T[g.L(k + 1, j, i)], T[g.L(kR, j, i)], u);
-    const double kap = kappa_eff(A, c, g.L(k + 1, j, i), ajc, dtde);
-    v = 0.0;
-    v += (g11 * dtdc + g21 * dtde + g31 * dtdz) * ajc * kap;
-}
-
-// One thread per local (ghosted) point; points off the reference's face loop get zero fluxes.
-__global__ void k_formt_faces(FormTArgs A, Geo g) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x - GW, j = blockIdx.y * blockDim.y + threadIdx.y - GW,
-              k = blockIdx.z - GW;
-    if (i >= g.mx + GW || j >= g.my + GW) return;
-    const long c = g.L(k, j, i);
-    V3 dv{0.0, 0.0, 0.0}, vs{0.0, 0.0, 0.0};
-    const bool in = i >= 0 && j >= 0 && k >= 0 && i < g.mx - 1 && j < g.my - 1 && k < g.mz - 1;
-    if (in) {
-        if (j != 0 && k != 0) flux_i(A, g, i, j, k, dv.x, vs.x);
-        if (i != 0 && k != 0) flux_j(A, g, i, j, k, dv.y, vs.y);
-        if (i != 0 && j != 0) flux_k(A, g, i, j, k, dv.z, vs.z);
-    }
-    st3(A.div, c, dv);
-    st3(A.visc, c, vs);
-}
-
+// ------------------------------------------------------------------------------------------------
+// Face fluxes, their budgets and the cell Jacobian in one launch.  A workgroup of NR rows of 64 points
+// (lane 0 and row 0 only supply their + faces) marches along k: the i face below a cell comes from the
+// lane before, the j face from the row before through LDS (one barrier a plane, two buffers) and the k
+// face from the plane before, in registers.  Face 0 of a periodic axis is evaluated as face m-2, which
+// resetFacePeriodicFluxesVector copies there.
+// Bound by the loads: 288 bytes a point at 4.1 TB/s, with about 950 L1 lines a wave and plane (nine vectors
+// at a stride of 24 bytes); the closure is a template parameter because the constants of pow(), kept in
+// registers across the planes, take a k_t model from 113 registers (four waves a SIMD) to 166 (1.22 ms).
+// 384 x 256 x 128, k_t: 1.24 ms as a face kernel that stored both fluxes of every face (0.95), twelve ghost
+// launches on them and a budget kernel, 1.06 so; 1.28 against 1.36 with nu_t.  Rows of 4 or 16 measured 1.09
+// and 1.10, loads without branches (195 registers) 1.24.
 // rhs = scale ((formMode != 2 ? div budget : 0) + (formMode != 1 ? visc budget : 0)) aj, interior
 // cells only (the reference writes nothing else of Rhs)
-__global__ void k_formt_cells(const double *div, const double *visc, const double *aj, double *rhs, double scale,
-                              int mode, Geo g) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x + 1, j = blockIdx.y * blockDim.y + threadIdx.y + 1,
-              k = blockIdx.z + 1;
-    if (i > g.mx - 2 || j > g.my - 2 || k > g.mz - 2) return;
-    const long c = g.L(k, j, i), ci = g.L(k, j, i - 1), cj = g.L(k, j - 1, i), ck = g.L(k - 1, j, i);
-    const double divBudget = div[3 * c] - div[3 * ci] + div[3 * c + 1] - div[3 * cj + 1] + div[3 * c + 2] - div[3 * ck + 2];
-    const double viscBudget =
-        visc[3 * c] - visc[3 * ci] + visc[3 * c + 1] - visc[3 * cj + 1] + visc[3 * c + 2] - visc[3 * ck + 2];
-    rhs[g.G(k, j, i)] = scale * ((mode != 2 ? divBudget : 0.0) + (mode != 1 ? viscBudget : 0.0)) * aj[c];
+// ------------------------------------------------------------------------------------------------
+constexpr int FT_NR = 8, FT_TI = 63, FT_TJ = FT_NR - 1;
+
+template <int KAP>
+__global__ void __launch_bounds__(64 * FT_NR) k_formt(FormTArgs A, Geo g, int kchunk) {
+    __shared__ double sJ[2][2][FT_NR][64];             // j-face fluxes (advective, diffusive) of the plane
+    const int lane = threadIdx.x, r = threadIdx.y;
+    const int tile = xcd_tile();                       // j fastest, then i, then the k chunk
+    const int bj = tile % gridDim.y, bi = (tile / gridDim.y) % gridDim.x, bk = tile / (gridDim.x * gridDim.y);
+    const int i = bi * FT_TI + lane, j = bj * FT_TJ + r;
+    const int kb = 1 + bk * kchunk, ke = min(kb + kchunk, g.mz - 1);      // cells [kb, ke)
+    const bool colI = i >= 1 && i <= g.mx - 2, colJ = j >= 1 && j <= g.my - 2;
+    const bool needI = r >= 1 && colJ && i <= g.mx - 2, needJ = lane >= 1 && colI && j <= g.my - 2;
+    const bool cell = lane >= 1 && r >= 1 && colI && colJ;
+    const int fi = (i == 0 && !g.nonper(0)) ? g.mx - 2 : i, fj = (j == 0 && !g.nonper(1)) ? g.my - 2 : j;
+    double dKm = 0.0, vKm = 0.0;                       // the k face below the cell
+    if (cell) {
+        const int kf = (kb == 1 && !g.nonper(2)) ? g.mz - 2 : kb - 1;
+        face_flux<2, KAP>(A, g, i, j, kf, g.L(kf, j, i), dKm, vKm);
+    }
+    for (int k = kb; k < ke; k++) {
+        const int buf = k & 1, ci = opaque_index(g.L(k, j, fi)), cj = opaque_index(g.L(k, fj, i)), c = opaque_index(g.L(k, j, i));
+        double dI = 0.0, vI = 0.0, dJ = 0.0, vJ = 0.0, dK = 0.0, vK = 0.0;
+        if (needJ) face_flux<1, KAP>(A, g, i, fj, k, cj, dJ, vJ);
+        sJ[buf][0][r][lane] = dJ; sJ[buf][1][r][lane] = vJ;
+        if (needI) face_flux<0, KAP>(A, g, fi, j, k, ci, dI, vI);
+        if (cell) face_flux<2, KAP>(A, g, i, j, k, c, dK, vK);
+        const double dIm = shup(dI), vIm = shup(vI);
+        __syncthreads();
+        if (cell) {
+            const double dJm = sJ[buf][0][r - 1][lane], vJm = sJ[buf][1][r - 1][lane];
+            const double divBudget = dI - dIm + dJ - dJm + dK - dKm, viscBudget = vI - vIm + vJ - vJm + vK - vKm;
+            A.rhs[g.G(k, j, i)] = A.scale * ((A.mode != 2 ? divBudget : 0.0) + (A.mode != 1 ? viscBudget : 0.0)) *
+                                  A.aj[c];
+        }
+        dKm = dK; vKm = vK;
+    }
 }
 
 bool kt_model(int m) {
@@ -266,29 +207,24 @@ FormTArgs formt_args(const Geo &g, const tosca_mesh *m, const tosca_params *p, c
     A.kcsi = m->kcsi; A.keta = m->keta; A.kzet = m->kzet;
     A.iaj = m->iaj; A.jaj = m->jaj; A.kaj = m->kaj;
     A.qI = tp->q_wall_i; A.qJ = tp->q_wall_j;
-    A.div = nullptr; A.visc = nullptr;
+    A.aj = m->aj; A.rhs = nullptr;
     A.nu = p->nu; A.pr = tp->pr; A.tref = p->t_ref;
-    A.les = p->les_active != 0;
-    A.ktm = A.les && kt_model(p->les_model);
     for (int q = 0; q < 4; q++) A.wall[q] = tp->wall_t[q];
     return A;
 }
 }  // namespace
 
-void ref_formt(const Geo &g, const tosca_mesh *m, const tosca_params *p, const tosca_teqn_params *tp,
-               const double *ucont, const double *theta, const double *nut, const double *kt, double *rhs,
-               double scale, int mode, double *ws, hipStream_t s) {
-    const long n = g.nloc();
+void formt(const Geo &g, const tosca_mesh *m, const tosca_params *p, const tosca_teqn_params *tp,
+           const double *ucont, const double *theta, const double *nut, const double *kt, double *rhs,
+           double scale, int mode, hipStream_t s) {
     FormTArgs A = formt_args(g, m, p, tp, ucont, theta, nut, kt);
-    A.div = ws; A.visc = ws + 3 * n;
-    const dim3 blk(64, 4, 1);
-    TOSCA_LAUNCH("k_formt_faces", k_formt_faces, dim3((g.gxm + 63) / 64, (g.gym + 3) / 4, g.gzm), blk, 0, s, A, g);
-    launch_wrap(A.div, 3, g, s);
-    launch_wrap(A.visc, 3, g, s);
-    launch_reset_face_periodic(A.div, 3, g, s);
-    launch_reset_face_periodic(A.visc, 3, g, s);
-    TOSCA_LAUNCH("k_formt_cells", k_formt_cells, dim3((g.mx - 2 + 63) / 64, (g.my - 2 + 3) / 4, g.mz - 2), blk, 0, s,
-                 A.div, A.visc, m->aj, rhs, scale, mode, g);
+    A.rhs = rhs; A.scale = scale; A.mode = mode;
+    const int ti = (g.mx - 2 + FT_TI - 1) / FT_TI, tj = (g.my - 2 + FT_TJ - 1) / FT_TJ;
+    const int kc = plane_chunk(g.mz - 2, ti * tj, 2 * NUM_CU, 1, 500.0);
+    const dim3 grid(ti, tj, (g.mz - 2 + kc - 1) / kc), block(64, FT_NR);
+    if (!p->les_active) TOSCA_LAUNCH("k_formt", k_formt<KAP_NONE>, grid, block, 0, s, A, g, kc);
+    else if (kt_model(p->les_model)) TOSCA_LAUNCH("k_formt", k_formt<KAP_KT>, grid, block, 0, s, A, g, kc);
+    else TOSCA_LAUNCH("k_formt", k_formt<KAP_NUT>, grid, block, 0, s, A, g, kc);
 }
 
 }  // namespace tosca

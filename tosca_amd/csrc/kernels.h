@@ -75,10 +75,10 @@ void launch_temperature_bcs(double *t, const int *bc_t, const double *t_value, c
 // GradP (gradp.hip): dp (global vector) from the local pressure p
 void launch_grad_p(const double *p, const tosca_mesh *m, double *dp, const Geo &g, hipStream_t s);
 
-// FormT (formt.hip): reference-structured face and cell kernels; ws holds 6 local doubles per point
-void ref_formt(const Geo &g, const tosca_mesh *m, const tosca_params *p, const tosca_teqn_params *tp,
-               const double *ucont, const double *theta, const double *nut, const double *kt, double *rhs,
-               double scale, int mode, double *ws, hipStream_t s);
+// FormT (formt.hip)
+void formt(const Geo &g, const tosca_mesh *m, const tosca_params *p, const tosca_teqn_params *tp, const double *ucont,
+           const double *theta, const double *nut, const double *kt, double *rhs, double scale, int mode,
+           hipStream_t s);
 
 // wind-farm body force (farm.hip): projectBladeForce's uniformADM branch into the local scat, and
 // bodyForceCartesian2Contravariant into the global scont
