@@ -285,16 +285,11 @@ void queue_step(tosca_ctx *c, const tosca_mesh *m, const tosca_params *p, const 
     } else if (p->les_model == TOSCA_LES_DPASD) {
         tosca::fused_dpasd<T>(g, m, ucat, p->max_cs, cs, nut, ws, s);
     } else {
-        tosca::launch_fill(cs, (long)g.nloc(), 0.0289, s);   // VecSet(lCs, std_cs), les.c:172-179
-        tosca::fused_nut<T>(g, m, ucat, cs, nut, nullptr, s);
+        tosca::fused_nut<T>(g, m, ucat, cs, nut, nullptr, s, cs, 0.0289);    // VecSet(lCs, std_cs), les.c:172-179
     }
-    if (p->les_model == TOSCA_LES_DSM || p->les_model == TOSCA_LES_DPASD) {
-        tosca::launch_wrap(cs, 1, g, s);
-        tosca::launch_reset_cell_periodic(cs, 1, g, s);
-    }
-    // UpdateNut: zero outside the interior, boundary conditions, ghost wrap
-    tosca::zero_outside_interior(nut, g, s);
-    tosca::nut_bcs(nut, p, g, s);
+    // UpdateNut: zero outside the interior, boundary conditions, ghost wrap; Cs there too
+    const bool dynamic = p->les_model == TOSCA_LES_DSM || p->les_model == TOSCA_LES_DPASD;
+    tosca::launch_nut_ghosts(nut, p, g, s, cs, dynamic ? -1.0 : 0.0289);
     // Buoyancy + FormU
     tosca::FormUArgsT<T, MT> A{};
     A.ucont = ucont; A.ucat = ucat; A.nut = nut;
@@ -444,8 +439,7 @@ void queue_imex(tosca_ctx *c, const tosca_mesh *m, const tosca_params *p, const 
     const Geo &g = c->geo;
     hipStream_t s = c->stream;
     const long ng3 = 3L * g.mx * g.my * g.mz;
-    tosca::launch_global_to_local(ucont, v, g, s);                         // :1763-1767
-    tosca::launch_wrap(ucont, 3, g, s);
+    tosca::launch_global_to_local(ucont, v, g, s);                         // :1763-1767 (wrapped below)
     tosca::launch_no_penetration(ucont, p, g, s);                          // :1770
     tosca::launch_reset_face_periodic(ucont, 3, g, s);                     // :1773
     tosca::launch_contra_to_cart(ucont, m, ucat, g, s);                    // :1777
@@ -893,9 +887,10 @@ int tosca_ueqn_rk4(tosca_ctx *c, const tosca_mesh *m, const tosca_params *p, dou
         queue_explicit(c, m, p, ucont, ucat, nut, dp, btheta, btheta_o, ab2, farm, ucont_o, rhs, form_mode);   // :1489
         // utmp += dt b_i Rhs (:1492) and, in the same pass, the next stage's ucont = Ucont_o +
         // a_{i+1} dt Rhs (:1480-1486) or, after the last stage, ucont = utmp (:1495-1497)
+        // (the next stage wraps ucont behind its resets, before anything reads its ghosts)
         tosca::launch_rk_stage(utmp, dt * b[i], rhs, ucont, i < 3 ? a[i + 1] * dt : 0.0, ucont_o, i == 3, g, s);
-        tosca::launch_wrap(ucont, 3, g, s);
     }
+    tosca::launch_wrap(ucont, 3, g, s);
     return launched(c, "UeqnRK4");
 }
 
@@ -925,9 +920,10 @@ void queue_rk3w(tosca_ctx *c, const tosca_mesh *m, const tosca_params *p, double
         if (chk) tosca::launch_local_to_global(chk + st * ng3, ucont, g, s);
         queue_explicit(c, m, p, ucont, ucat, nut, dp, btheta, btheta_o, ab2, farm, ucont_o, rhs, form_mode);   // :1527
         // Ucont = (Ucont + dt beta_i Rhs) + (-1.0 dt delta_i) Rhs_o; Rhs_o = Rhs (:1533-1541, 1563-1569)
+        // (the next stage wraps ucont behind its resets, before anything reads its ghosts)
         tosca::launch_rk3w_update(ucont, rhs, rhs_o, dt * kWrayBeta[i], -1.0 * dt * kWrayDelta[i], g, s);
-        tosca::launch_wrap(ucont, 3, g, s);
     }
+    if (n_stages > 0) tosca::launch_wrap(ucont, 3, g, s);
     if (chk) tosca::launch_local_to_global(chk + (long)n_stages * ng3, ucont, g, s);
 }
 
@@ -1001,7 +997,6 @@ int tosca_ueqn_rk3w_adjoint(tosca_ctx *c, const tosca_mesh *m, const tosca_param
         const double *x = chk + (size_t)st * ng3, *uo = chk + (size_t)(st - i) * ng3;
         // the stage's reset fluxes and Cartesian velocity, recomputed from its checkpoint
         tosca::launch_global_to_local(ucont, x, g, s);
-        tosca::launch_wrap(ucont, 3, g, s);
         tosca::launch_no_penetration(ucont, p, g, s);
         tosca::launch_reset_face_periodic(ucont, 3, g, s);
         tosca::launch_contra_to_cart(ucont, m, ucat, g, s);
@@ -1021,7 +1016,6 @@ int tosca_ueqn_rk3w_adjoint(tosca_ctx *c, const tosca_mesh *m, const tosca_param
     // leave ucont and ucat as the forward sweep left them
     if (n_stages > 0) {
         tosca::launch_global_to_local(ucont, chk + (size_t)(n_stages - 1) * ng3, g, s);
-        tosca::launch_wrap(ucont, 3, g, s);
         tosca::launch_no_penetration(ucont, p, g, s);
         tosca::launch_reset_face_periodic(ucont, 3, g, s);
         tosca::launch_contra_to_cart(ucont, m, ucat, g, s);
@@ -1216,8 +1210,7 @@ int tosca_snes_func_eval(tosca_ctx *c, const tosca_mesh *m, const tosca_params *
     if ((rc = check_dev(c, u, vb, "u")) || (rc = check_dev(c, bU, vb, "bU")) || (rc = check_dev(c, F, vb, "F"))) return rc;
     if (F == u || F == bU || F == ucont_o) return set_err(c, TOSCA_ERR_ARG, "F must not alias an input");
     hipStream_t s = c->stream;
-    tosca::launch_global_to_local(ucont, u, g, s);                           // :1195-1199
-    tosca::launch_wrap(ucont, 3, g, s);
+    tosca::launch_global_to_local(ucont, u, g, s);                           // :1195-1199 (wrapped below)
     tosca::launch_no_penetration(ucont, p, g, s);                            // :1202
     tosca::launch_reset_face_periodic(ucont, 3, g, s);                       // :1205
     tosca::launch_contra_to_cart(ucont, m, ucat, g, s);                      // :1208
@@ -1426,7 +1419,6 @@ int tosca_update_cs(tosca_ctx *c, const tosca_mesh *m, const tosca_params *p, co
     if (!c->ref_path && (p->les_model == TOSCA_LES_DSM || p->les_model == TOSCA_LES_DPASD)) {
         if (p->les_model == TOSCA_LES_DSM) tosca::fused_dsm<double>(c->geo, m, ucat, p->max_cs, cs, nullptr, c->ws, c->stream);
         else tosca::fused_dpasd<double>(c->geo, m, ucat, p->max_cs, cs, nullptr, c->ws, c->stream);
-        tosca::launch_wrap(cs, 1, c->geo, c->stream);
         tosca::launch_reset_cell_periodic(cs, 1, c->geo, c->stream);
     } else {
         tosca::ref_update_cs(c->geo, m, p, ucat, cs, c->ws, c->stream);
@@ -1450,10 +1442,8 @@ int tosca_update_nut(tosca_ctx *c, const tosca_mesh *m, const tosca_params *p, c
         tosca::ref_update_nut(c->geo, m, p, ucat, cs, nut, ksgs, c->stream);
     } else {
         tosca::fused_nut(c->geo, m, ucat, cs, nut, ksgs, c->stream);
-        tosca::zero_outside_interior(nut, c->geo, c->stream);
-        if (ksgs) tosca::zero_outside_interior(ksgs, c->geo, c->stream);
-        tosca::nut_bcs(nut, p, c->geo, c->stream);
-        if (ksgs) tosca::launch_wrap(ksgs, 1, c->geo, c->stream);
+        tosca::launch_nut_ghosts(nut, p, c->geo, c->stream);
+        if (ksgs) tosca::launch_nut_ghosts(ksgs, static_cast<const tosca_params *>(nullptr), c->geo, c->stream);
     }
     return launched(c, "UpdateNut");
 }

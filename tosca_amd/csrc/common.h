@@ -426,4 +426,41 @@ __device__ __forceinline__ int xcd_tile() {
     return xcd_tile(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), gridDim.x * gridDim.y * gridDim.z);
 }
 
+// The points of an outer box outside a core box, as six disjoint slabs: the low and the high k slab over
+// whole planes, the j slabs between them, the i slabs between those (thicknesses may be zero); thread t of
+// a launch over `total` threads takes point t.  (Written shells are thin: a launch costs about 4 us of host
+// and queue time whatever it writes, so every ghost operation is one launch, whose source index is the
+// composition of the operations along the axes.)
+struct Shell {
+    int end[6], i0[6], j0[6], k0[6], ni[6], nj[6];
+    int total;
+};
+inline Shell make_shell(const int (&olo)[3], const int (&ohi)[3], const int (&clo)[3], const int (&chi)[3]) {
+    Shell B;
+    int n = 0;
+    auto slab = [&](int q, int i0, int i1, int j0, int j1, int k0, int k1) {
+        const int ni = max(0, i1 - i0), nj = max(0, j1 - j0), nk = max(0, k1 - k0);
+        B.i0[q] = i0; B.j0[q] = j0; B.k0[q] = k0; B.ni[q] = ni; B.nj[q] = nj;
+        B.end[q] = n += ni * nj * nk;
+    };
+    slab(0, olo[0], ohi[0], olo[1], ohi[1], olo[2], clo[2]);
+    slab(1, olo[0], ohi[0], olo[1], ohi[1], chi[2], ohi[2]);
+    slab(2, olo[0], ohi[0], olo[1], clo[1], clo[2], chi[2]);
+    slab(3, olo[0], ohi[0], chi[1], ohi[1], clo[2], chi[2]);
+    slab(4, olo[0], clo[0], clo[1], chi[1], clo[2], chi[2]);
+    slab(5, chi[0], ohi[0], clo[1], chi[1], clo[2], chi[2]);
+    B.total = n;
+    return B;
+}
+__device__ __forceinline__ bool shell_point(const Shell &B, int t, int &i, int &j, int &k) {
+    if (t >= B.total) return false;
+    int q = 0, start = 0;
+    while (t >= B.end[q]) start = B.end[q++];
+    const int e = t - start, r = e / B.ni[q];
+    i = B.i0[q] + e % B.ni[q];
+    j = B.j0[q] + r % B.nj[q];
+    k = B.k0[q] + r / B.nj[q];
+    return true;
+}
+
 }  // namespace tosca

@@ -80,24 +80,8 @@ size_t dpasd_ws_doubles(const Geo &g);
 
 // nut = Cs Delta^2 |S| at interior cells from a given Cs (Smagorinsky, or any stored Cs)
 template <class T>
-void fused_nut(const Geo &g, const tosca_mesh *m, const T *ucat, const double *cs, T *nut, T *ksgs, hipStream_t s);
-
-// zero the shell of an nx*ny*nz array (ncomp values per point) outside its interior cells,
-// the interior being [1+lo, n-2-hi] on each axis in array coordinates
-template <class T>
-void zero_shell(T *a, int ncomp, int nx, int ny, int nz, int lo, int hi, hipStream_t s);
-
-// y += x (VecAXPY with a = 1) on the points of an nx*ny*nz vector array outside [1, n-2] on every
-// axis: the part of the wind-farm AXPY the fused FormU kernel does not cover
-void shell_add(double *y, const double *x, int nx, int ny, int nz, hipStream_t s);
-
-// zero every point of a local scalar array outside the interior cells
-template <class T>
-void zero_outside_interior(T *a, const Geo &g, hipStream_t s);
-
-// nut ghost cells: UpdateNutBCs subset + ghost wrap
-template <class T>
-void nut_bcs(T *nut, const tosca_params *p, const Geo &g, hipStream_t s);
+void fused_nut(const Geo &g, const tosca_mesh *m, const T *ucat, const double *cs, T *nut, T *ksgs, hipStream_t s,
+               double *cs_fill = nullptr, double fill = 0.0);
 
 // Adjoint of R = FormU(ucont, ucat, UpdateNut(ucat, cs)) + Buoyancy(theta): accumulates the
 // cotangents of the four inputs (overwritten) from rbar; ws holds vjp_ws_doubles(g) doubles.

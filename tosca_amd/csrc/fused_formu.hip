@@ -346,7 +346,7 @@ __global__ void __launch_bounds__(64 * NR) k_fused_formu(MainArgs<T, MT> A, Geo 
     const bool out = cell && lane <= TI && r <= TJ;
     // The last output row has no row above it in the tile: the j-face dot of its Rhs is split at
     // the seam.  It keeps the half of its own cell (v1) in sv1 and the next tile's first output
-    // row keeps the half of its cell (the same v2 this row would form) in sv2; k_formu_jseam adds
+    // row keeps the half of its cell (the same v2 this row would form) in sv2; k_formu_tail adds
     // both.  The domain's last interior row completes its dot here (own fp, or the periodic seam).
     const bool seamRow = r == NR - 1 && j < g.my - 2;
     const bool seamNext = r == 1 && bj > 0;
@@ -571,7 +571,7 @@ __global__ void __launch_bounds__(64 * NR) k_fused_formu(MainArgs<T, MT> A, Geo 
             const double rz = A.scale * fa2p * (0.5 * (v1 + v2));
             A.rhs[ro] = r0 + rx;
             if (!seamRow) A.rhs[ro + 1] = r1 + ry;
-            else if (A.farm) A.rhs[ro + 1] = r1;      // k_formu_jseam adds the dot to rhs + farm
+            else if (A.farm) A.rhs[ro + 1] = r1;      // k_formu_tail adds the dot to rhs + farm
             A.rhs[ro + 2] = r2 + rz;
             if (buoy) {
                 // Boussinesq source on the three + faces of the cell (ueqn_sources.c:2812-2870):
@@ -603,15 +603,27 @@ __global__ void __launch_bounds__(64 * NR) k_fused_formu(MainArgs<T, MT> A, Geo 
     }
 }
 
-// Rhs.y of the j-tile seam rows: rhs += scale aj_j (0.5 (v1 + v2)) with the two halves the main
-// kernel kept (the same expression, so the same value, as the other rows' in-kernel update)
+// What is left behind the main kernel, in one launch:
+//   Rhs.y of the j-tile seam rows: rhs += scale aj_j (0.5 (v1 + v2)) with the two halves the main
+//   kernel kept (the same expression, so the same value, as the other rows' in-kernel update);
+//   on the owned points outside the interior cells (the main kernel covers the interior) the farm AXPY
+//   (rhs += 1 farm) and bTheta = 0 (the reference zeroes all of it), either null
 template <class MT>
-__global__ void k_formu_jseam(double *rhs, const double *sv1, const double *sv2, const MT *jaj, double scale, Geo g,
-                              int tj) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y, sidx = blockIdx.z;
+__global__ void __launch_bounds__(256) k_formu_tail(double *rhs, const double *sv1, const double *sv2, const MT *jaj, double scale,
+                                                    Geo g, int tj, int seams, const double *farm, double *btheta, Shell S) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= seams) {
+        int i, j, k;
+        if (!shell_point(S, t - seams, i, j, k)) return;
+        const int o = 3 * g.G(k, j, i);
+        if (farm) { rhs[o] = rhs[o] + 1.0 * farm[o]; rhs[o + 1] = rhs[o + 1] + 1.0 * farm[o + 1]; rhs[o + 2] = rhs[o + 2] + 1.0 * farm[o + 2]; }
+        if (btheta) { btheta[o] = 0.0; btheta[o + 1] = 0.0; btheta[o + 2] = 0.0; }
+        return;
+    }
+    const int i = t % g.mx, k = t / g.mx % g.mz, sidx = t / (g.mx * g.mz);
     const int jA = (sidx + 1) * tj;                 // last output row of j tile sidx
     if (i < 1 || i > g.mx - 2 || k < 1 || k > g.mz - 2 || jA >= g.my - 2) return;
-    const long o = ((long)sidx * g.mz + k) * g.mx + i;
+    const int o = (sidx * g.mz + k) * g.mx + i;
     const double fa = jaj[g.L(k, jA, i)];
     double *pr = rhs + 3 * (long)g.G(k, jA, i) + 1;
     *pr = *pr + scale * fa * (0.5 * (sv1[o] + sv2[o]));
@@ -663,13 +675,15 @@ void fused_formu(const Geo &g, const FormUArgsT<T, MT> &A, double *ws, hipStream
         if (derive) TOSCA_LAUNCH(kname, (k_fused_formu<NR, T, MT, true>), grid, dim3(64, NR), 0, s, M, g, kchunk);
     }
     if (!derive) TOSCA_LAUNCH(kname, (k_fused_formu<NR, T, MT, false>), grid, dim3(64, NR), 0, s, M, g, kchunk);
-    // the farm AXPY on the owned points outside the interior cells (the kernel covers the interior)
-    if (A.farm) shell_add(A.rhs, A.farm, g.mx, g.my, g.mz, s);
-    if (nsj > 1)
-        TOSCA_LAUNCH("k_formu_jseam", k_formu_jseam<MT>, dim3((g.mx + 127) / 128, g.mz, nsj - 1), dim3(128), 0, s,
-                     A.rhs, sv1, sv2, A.jaj, A.scale, g, TJ);
-    // the reference zeroes all of bTheta; the kernel writes the interior cells, this the rest
-    if (A.btheta) zero_shell(A.btheta, 3, g.mx, g.my, g.mz, 0, 0, s);
+    const int seams = (nsj - 1) * g.mz * g.mx;
+    Shell S{};
+    if (A.farm || A.btheta) {
+        const int zero[3] = {0, 0, 0}, own[3] = {g.mx, g.my, g.mz}, lo[3] = {1, 1, 1}, hi[3] = {g.mx - 1, g.my - 1, g.mz - 1};
+        S = make_shell(zero, own, lo, hi);
+    }
+    if (seams + S.total)
+        TOSCA_LAUNCH("k_formu_tail", k_formu_tail<MT>, dim3((seams + S.total + 255) / 256), dim3(256), 0, s, A.rhs, sv1, sv2, A.jaj,
+                     A.scale, g, TJ, seams, A.farm, A.btheta, S);
 }
 
 template void fused_formu<double, double>(const Geo &, const FormUArgsT<double, double> &, double *, hipStream_t);

@@ -613,7 +613,7 @@ __global__ void __launch_bounds__(CX * CY) k_dsm_cs_nut(Geo g, const double *LM,
 
 template <class T>
 __global__ void __launch_bounds__(256) k_nut_fused(Geo g, const T *ucat, const double *csi, const double *eta, const double *zet,
-                            const double *aj, const double *Cs, T *nut, T *ksgs) {
+                            const double *aj, const double *Cs, T *nut, T *ksgs, double *csw, double csv) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1, j = blockIdx.y * blockDim.y + threadIdx.y + 1,
               k = blockIdx.z + 1;
     if (i > g.mx - 2 || j > g.my - 2 || k > g.mz - 2) return;
@@ -622,7 +622,9 @@ __global__ void __launch_bounds__(256) k_nut_fused(Geo g, const T *ucat, const d
     const double a = aj[c];
     const double S = strain_mag(du_dxyz(cvt3<T>(cc), cvt3<T>(ee), cvt3<T>(zz), T(a), du_center(g, ucat, i, j, k)));
     const double filter = cube_root(1. / a);
-    const double nt = Cs[c] * (filter * filter) * S;      // pow(x, 2.) of les.c:2510 is x * x, exactly rounded
+    const double cs = csw ? csv : Cs[c];
+    if (csw) csw[c] = csv;
+    const double nt = cs * (filter * filter) * S;      // pow(x, 2.) of les.c:2510 is x * x, exactly rounded
     nut[c] = T(nt);
     if (ksgs) {
         const double V = 1.0 / a;
@@ -855,73 +857,6 @@ __global__ void __launch_bounds__(256) k_dpasd_cs_nut(Geo g, const double *csP, 
     }
 }
 
-// zero six disjoint boxes of an array with row length nx and plane size nx*ny (ncomp values per
-// point) in one launch: blockIdx.y selects the box, the blocks stride over its values
-struct ShellBoxes { int i0[6], j0[6], k0[6], ni[6], nj[6], nk[6]; };
-
-template <class T>
-__global__ void k_zero_box(T *a, int ncomp, int nx, int ny, ShellBoxes B) {
-    const int b = blockIdx.y;
-    if (B.ni[b] <= 0 || B.nj[b] <= 0 || B.nk[b] <= 0) return;
-    const long row = (long)B.ni[b] * ncomp, tot = row * B.nj[b] * B.nk[b];
-    for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < tot; t += (long)gridDim.x * blockDim.x) {
-        const long e = t % row, r = t / row;
-        const int jj = (int)(r % B.nj[b]), kk = (int)(r / B.nj[b]);
-        const long p = ((long)(B.k0[b] + kk) * ny + (B.j0[b] + jj)) * nx + B.i0[b];
-        a[p * ncomp + e] = T(0);
-    }
-}
-
-template <class T>
-void zero_shell(T *a, int ncomp, int nx, int ny, int nz, int lo, int hi, hipStream_t s) {
-    // boxes (in array coordinates) covering everything but [lo+1 .. n-hi-2] on every axis:
-    // `lo` / `hi` extra layers outside the boundary cells on the low / high side
-    const int w0 = lo + 1, w1 = hi + 1;            // shell thickness per side
-    ShellBoxes B{};
-    auto box = [&](int q, int i0, int j0, int k0, int ni, int nj, int nk) {
-        B.i0[q] = i0; B.j0[q] = j0; B.k0[q] = k0; B.ni[q] = ni; B.nj[q] = nj; B.nk[q] = nk;
-    };
-    box(0, 0, 0, 0, nx, ny, w0);                                   // low k slab
-    box(1, 0, 0, nz - w1, nx, ny, w1);                             // high k slab
-    box(2, 0, 0, w0, nx, w0, nz - w0 - w1);                        // low j slab
-    box(3, 0, ny - w1, w0, nx, w1, nz - w0 - w1);                  // high j slab
-    box(4, 0, w0, w0, w0, ny - w0 - w1, nz - w0 - w1);             // low i slab
-    box(5, nx - w1, w0, w0, w1, ny - w0 - w1, nz - w0 - w1);       // high i slab
-    TOSCA_LAUNCH("k_zero_box", k_zero_box<T>, dim3(512, 6), dim3(256), 0, s, a, ncomp, nx, ny, B);
-}
-
-// y = y + 1 x over the same six boxes (three values per point)
-__global__ void k_add_box(double *y, const double *x, int nx, int ny, ShellBoxes B) {
-    const int b = blockIdx.y;
-    if (B.ni[b] <= 0 || B.nj[b] <= 0 || B.nk[b] <= 0) return;
-    const long row = (long)B.ni[b] * 3, tot = row * B.nj[b] * B.nk[b];
-    for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < tot; t += (long)gridDim.x * blockDim.x) {
-        const long e = t % row, r = t / row;
-        const int jj = (int)(r % B.nj[b]), kk = (int)(r / B.nj[b]);
-        const long p = ((long)(B.k0[b] + kk) * ny + (B.j0[b] + jj)) * nx + B.i0[b];
-        y[p * 3 + e] = y[p * 3 + e] + 1.0 * x[p * 3 + e];
-    }
-}
-
-void shell_add(double *y, const double *x, int nx, int ny, int nz, hipStream_t s) {
-    ShellBoxes B{};
-    auto box = [&](int q, int i0, int j0, int k0, int ni, int nj, int nk) {
-        B.i0[q] = i0; B.j0[q] = j0; B.k0[q] = k0; B.ni[q] = ni; B.nj[q] = nj; B.nk[q] = nk;
-    };
-    box(0, 0, 0, 0, nx, ny, 1);
-    box(1, 0, 0, nz - 1, nx, ny, 1);
-    box(2, 0, 0, 1, nx, 1, nz - 2);
-    box(3, 0, ny - 1, 1, nx, 1, nz - 2);
-    box(4, 0, 1, 1, 1, ny - 2, nz - 2);
-    box(5, nx - 1, 1, 1, 1, ny - 2, nz - 2);
-    TOSCA_LAUNCH("k_add_box", k_add_box, dim3(256, 6), dim3(256), 0, s, y, x, nx, ny, B);
-}
-
-template <class T>
-void zero_outside_interior(T *a, const Geo &g, hipStream_t s) {
-    zero_shell(a, 1, g.gxm, g.gym, g.gzm, GW, GW, s);
-}
-
 namespace {
 // launch shape of k_les_filter<H>, which also sizes DPASD's partials
 struct FilterShape { int ti, tj, chunks, kchunk; };
@@ -1046,24 +981,19 @@ void fused_dsm(const Geo &g, const tosca_mesh *m, const T *ucat, double maxCs, d
 }
 
 template <class T>
-void fused_nut(const Geo &g, const tosca_mesh *m, const T *ucat, const double *cs, T *nut, T *ksgs, hipStream_t s) {
+void fused_nut(const Geo &g, const tosca_mesh *m, const T *ucat, const double *cs, T *nut, T *ksgs, hipStream_t s, double *cs_fill,
+               double fill) {
     TOSCA_LAUNCH(sizeof(T) == 8 ? "k_nut_fused" : "k_nut_fused_f32", k_nut_fused<T>, dim3((g.mx - 2 + 63) / 64, (g.my - 2 + 3) / 4, g.mz - 2), dim3(64, 4), 0,
-                 s, g, ucat, m->csi, m->eta, m->zet, m->aj, cs, nut, ksgs);
+                 s, g, ucat, m->csi, m->eta, m->zet, m->aj, cs, nut, ksgs, cs_fill, fill);
 }
 
-template <class T>
-void nut_bcs(T *nut, const tosca_params *p, const Geo &g, hipStream_t s) { launch_nut_bcs(nut, p, g, s); }
-
 #define TOSCA_LES_INSTANTIATE(T)                                                                            \
-    template void zero_shell<T>(T *, int, int, int, int, int, int, hipStream_t);                            \
-    template void zero_outside_interior<T>(T *, const Geo &, hipStream_t);                                  \
     template void fused_dsm<T>(const Geo &, const tosca_mesh *, const T *, double, double *, T *, double *,   \
                                hipStream_t, const tosca_mesh_f32 *);                                         \
     template void fused_dpasd<T>(const Geo &, const tosca_mesh *, const T *, double, double *, T *, double *, \
                                  hipStream_t);                                                               \
     template void fused_nut<T>(const Geo &, const tosca_mesh *, const T *, const double *, T *, T *,         \
-                               hipStream_t);                                                                 \
-    template void nut_bcs<T>(T *, const tosca_params *, const Geo &, hipStream_t);
+                               hipStream_t, double *, double);
 TOSCA_LES_INSTANTIATE(double)
 TOSCA_LES_INSTANTIATE(float)
 

@@ -6,12 +6,16 @@
 
 namespace tosca {
 
-// ghost handling (ref_kernels.hip)
+// ghost handling (ref_kernels.hip), one launch each: the wraps of the periodic axes alone, after
+// resetCellPeriodicFluxes, after resetFacePeriodicFluxesVector; and nu_t outside the interior cells
 template <class T> void launch_wrap(T *a, int ncomp, const Geo &g, hipStream_t s);
 void launch_reset_cell_periodic(double *a, int ncomp, const Geo &g, hipStream_t s);
 void launch_reset_face_periodic(double *a, int ncomp, const Geo &g, hipStream_t s);
 void launch_fill(double *a, long n, double v, hipStream_t s);
-template <class T> void launch_nut_bcs(T *nut, const tosca_params *p, const Geo &g, hipStream_t s);
+// (p null: no patch kinds, as for a scalar that is zero there); cs given: in the same launch Cs outside the
+// interior, the constant cs_fill or (< 0) its periodic resets and wraps
+template <class T> void launch_nut_ghosts(T *nut, const tosca_params *p, const Geo &g, hipStream_t s, double *cs = nullptr,
+                                          double cs_fill = -1.0);
 
 // reference-structured path (ref_kernels.hip); `ws` is a workspace of >= 22 * nloc doubles
 void ref_formu(const Geo &g, const tosca_mesh *m, const tosca_params *p, const double *ucont, const double *ucat,

@@ -6,10 +6,10 @@
 //   FormU       src/solvers/ueqn_solvers.c:6-1083   -> k_formu_faces, k_formu_cells, k_formu_dot
 //   UpdateCs    src/les.c:165-2115                  -> k_strain, k_test_filter<3|5>, k_box_clip,
 //                                                      k_plane_partial/k_plane_final/k_dpasd_cs
-//   UpdateNut   src/les.c:2119-2578 + boundary.c:2630-2929 -> k_nut, k_nut_bc
+//   UpdateNut   src/les.c:2119-2578 + boundary.c:2630-2929 -> k_nut, k_nut_ghosts
 //   Buoyancy    src/sources/ueqn_sources.c:2726-2880 -> k_buoyancy
 //   ghost scatters (PETSc DMLocalToLocal), resetCellPeriodicFluxes and
-//   resetFacePeriodicFluxesVector -> k_wrap_axis, k_reset_axis
+//   resetFacePeriodicFluxesVector -> k_ghosts
 #include "kernels.h"
 
 namespace tosca {
@@ -17,42 +17,29 @@ namespace tosca {
 // ---------------------------------------------------------------------------------------------
 // ghost handling
 // ---------------------------------------------------------------------------------------------
-// DMLocalToLocal along one DM_BOUNDARY_PERIODIC axis: ghost slabs take the wrapped owned values.
-// The transverse ranges cover the ghosts of periodic-wrap axes and the owned range otherwise.
-template <class T>
-__global__ void k_wrap_axis(T *a, int ncomp, Geo g, int axis) {
-    const int m[3] = {g.mx, g.my, g.mz};
-    int t1 = (axis == 0) ? 1 : 0, t2 = (axis == 2) ? 1 : 2;
-    int lo1 = (g.per[t1] == TOSCA_PERIODIC_WRAP) ? -GW : 0, n1 = m[t1] + ((g.per[t1] == TOSCA_PERIODIC_WRAP) ? 2 * GW : 0);
-    int lo2 = (g.per[t2] == TOSCA_PERIODIC_WRAP) ? -GW : 0, n2 = m[t2] + ((g.per[t2] == TOSCA_PERIODIC_WRAP) ? 2 * GW : 0);
-    int a1 = blockIdx.x * blockDim.x + threadIdx.x;
-    int a2 = blockIdx.y;
-    int s = blockIdx.z;                   // 0..2*GW-1: which ghost layer
-    if (a1 >= n1 || a2 >= n2) return;
-    int n = m[axis];
-    int dst = (s < GW) ? (s - GW) : (n + s - GW);       // -3..-1, n..n+2
-    int src = (s < GW) ? (n + s - GW) : (s - GW);       // n-3..n-1, 0..2
-    int idx_d[3], idx_s[3];
-    idx_d[axis] = dst; idx_s[axis] = src;
-    idx_d[t1] = idx_s[t1] = lo1 + a1;
-    idx_d[t2] = idx_s[t2] = lo2 + a2;
-    int cd = g.L(idx_d[2], idx_d[1], idx_d[0]), cs = g.L(idx_s[2], idx_s[1], idx_s[0]);
-    for (int q = 0; q < ncomp; q++) a[ncomp * cd + q] = a[ncomp * cs + q];
+// DMLocalToLocal on the DM_BOUNDARY_PERIODIC axes (ghost layers take the wrapped owned values; the other
+// axes keep their ghosts), after the periodic resets of `reset` (src/include/inline.h):
+//   RESET_CELL  resetCellPeriodicFluxes (:5496-5514): the boundary cells 0 / m-1 of a periodic axis take
+//               cells m-2 / 1 over the whole owned range of the other two axes
+//   RESET_FACE  resetFacePeriodicFluxesVector (:5357-5451): the points of index 0 take the values at m-2
+//               (type 1; type 2 reads ghost -2, which holds m-2)
+// one axis after the other.  A written point's source is no written point, so the axes compose.
+enum { RESET_NONE, RESET_FACE, RESET_CELL };
+__device__ __forceinline__ int ghost_source(int x, int m, int per, int reset) {
+    if (per == TOSCA_PERIODIC_NONE) return x;
+    if (per == TOSCA_PERIODIC_WRAP) x = x < 0 ? x + m : x >= m ? x - m : x;
+    if (reset != RESET_NONE && x == 0) return m - 2;
+    if (reset == RESET_CELL && x == m - 1) return 1;
+    return x;
 }
-
-// resetCellPeriodicFluxes along one periodic axis: boundary ghost cells 0 / m-1 take cells
-// m-2 / 1 over the whole owned range of the other two axes (src/include/inline.h:5496-5514).
-__global__ void k_reset_axis(double *a, int ncomp, Geo g, int axis) {
-    const int m[3] = {g.mx, g.my, g.mz};
-    int t1 = (axis == 0) ? 1 : 0, t2 = (axis == 2) ? 1 : 2;
-    int a1 = blockIdx.x * blockDim.x + threadIdx.x, a2 = blockIdx.y, side = blockIdx.z;
-    if (a1 >= m[t1] || a2 >= m[t2]) return;
-    int idx_d[3], idx_s[3];
-    idx_d[axis] = side ? m[axis] - 1 : 0;
-    idx_s[axis] = side ? 1 : m[axis] - 2;
-    idx_d[t1] = idx_s[t1] = a1;
-    idx_d[t2] = idx_s[t2] = a2;
-    int cd = g.L(idx_d[2], idx_d[1], idx_d[0]), cs = g.L(idx_s[2], idx_s[1], idx_s[0]);
+__device__ __forceinline__ int ghost_point(const Geo &g, int i, int j, int k, int reset) {
+    return g.L(ghost_source(k, g.mz, g.per[2], reset), ghost_source(j, g.my, g.per[1], reset), ghost_source(i, g.mx, g.per[0], reset));
+}
+template <class T>
+__global__ void __launch_bounds__(256) k_ghosts(T *a, int ncomp, Geo g, Shell B, int reset) {
+    int i, j, k;
+    if (!shell_point(B, blockIdx.x * blockDim.x + threadIdx.x, i, j, k)) return;
+    const int cd = g.L(k, j, i), cs = ghost_point(g, i, j, k, reset);
     for (int q = 0; q < ncomp; q++) a[ncomp * cd + q] = a[ncomp * cs + q];
 }
 
@@ -424,26 +411,43 @@ __global__ void k_nut(const double *ucat, const double *csi, const double *eta, 
 
 struct NutBC { int bc[6]; double val[6]; };
 
-// UpdateNutBCs (boundary.c:2812-2917) along one axis: ghost cells next to the interior cells of
-// both patches of `axis`.  Reads interior values only.
+// nu_t (or another scalar, no patch kind given) outside the interior cells, from the interior ones: zero, then UpdateNutBCs (boundary.c:2812-2917)
+// on the ghost cells next to the interior cells of the six patches, then the wrapped ghost layers.  In the
+// same launch Cs: the constant `fill` at the same points, or (fill < 0) its periodic resets and wraps over
+// the points of C
 template <class T>
-__global__ void k_nut_bc(T *nut, NutBC B, Geo g, int axis) {
-    const int m[3] = {g.mx, g.my, g.mz};
-    int t1 = (axis == 0) ? 1 : 0, t2 = (axis == 2) ? 1 : 2;
-    int a1 = blockIdx.x * blockDim.x + threadIdx.x + 1, a2 = blockIdx.y + 1, side = blockIdx.z;
-    if (a1 >= m[t1] - 1 || a2 >= m[t2] - 1) return;
-    int patch = 2 * axis + side, n = m[axis];
-    int idx[3], src[3];
-    idx[t1] = src[t1] = a1;
-    idx[t2] = src[t2] = a2;
-    idx[axis] = side ? n - 1 : 0;
-    int bc = B.bc[patch];
-    T v;
-    if (bc == TOSCA_BCNUT_ZEROGRADIENT) { src[axis] = side ? n - 2 : 1; v = nut[g.L(src[2], src[1], src[0])]; }
-    else if (bc == TOSCA_BCNUT_FIXEDVALUE) v = T(B.val[patch]);
-    else if (bc == TOSCA_BCNUT_PERIODIC && g.per[axis] != TOSCA_PERIODIC_NONE) { src[axis] = side ? 1 : n - 2; v = nut[g.L(src[2], src[1], src[0])]; }
-    else return;
-    nut[g.L(idx[2], idx[1], idx[0])] = v;
+__global__ void __launch_bounds__(256) k_nut_ghosts(T *nut, NutBC B, Geo g, Shell S, double *cs, double fill, Shell C) {
+    int x[3];
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= S.total) {
+        if (shell_point(C, t - S.total, x[0], x[1], x[2])) cs[g.L(x[2], x[1], x[0])] = cs[ghost_point(g, x[0], x[1], x[2], RESET_CELL)];
+        return;
+    }
+    shell_point(S, t, x[0], x[1], x[2]);
+    const int c = g.L(x[2], x[1], x[0]), m[3] = {g.mx, g.my, g.mz};
+    if (fill >= 0.0) cs[c] = fill;
+    int outside = 0, axis = 0;               // of the owned point behind this one
+    bool owned = true;
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        x[q] = ghost_source(x[q], m[q], g.per[q], RESET_NONE);
+        owned = owned && x[q] >= 0 && x[q] < m[q];
+        if (x[q] == 0 || x[q] == m[q] - 1) { outside++; axis = q; }
+    }
+    T v = T(0);
+    if (owned && outside <= 1) {
+        bool read = outside == 0;
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+            if (outside == 0 || q != axis) continue;
+            const int side = x[q] != 0, bc = B.bc[2 * q + side];
+            if (bc == TOSCA_BCNUT_ZEROGRADIENT) { x[q] = side ? m[q] - 2 : 1; read = true; }
+            else if (bc == TOSCA_BCNUT_FIXEDVALUE) v = T(B.val[2 * q + side]);
+            else if (bc == TOSCA_BCNUT_PERIODIC && g.per[q] != TOSCA_PERIODIC_NONE) { x[q] = side ? 1 : m[q] - 2; read = true; }
+        }
+        if (read) v = nut[g.L(x[2], x[1], x[0])];
+    }
+    nut[c] = v;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -485,42 +489,32 @@ __global__ void k_buoyancy(const double *tmprt, const double *icsi, const double
 static inline dim3 blk2() { return dim3(64, 4, 1); }
 static inline dim3 grd(int ni, int nj, int nk) { return dim3((ni + 63) / 64, (nj + 3) / 4, nk); }
 
-template <class T>
-void launch_wrap(T *a, int ncomp, const Geo &g, hipStream_t s) {
+namespace {
+// the points k_ghosts writes
+Shell ghost_shell(const Geo &g, int reset) {
     const int m[3] = {g.mx, g.my, g.mz};
-    for (int axis = 0; axis < 3; axis++) {
-        if (g.per[axis] != TOSCA_PERIODIC_WRAP) continue;
-        int t1 = (axis == 0) ? 1 : 0, t2 = (axis == 2) ? 1 : 2;
-        int n1 = m[t1] + ((g.per[t1] == TOSCA_PERIODIC_WRAP) ? 2 * GW : 0);
-        int n2 = m[t2] + ((g.per[t2] == TOSCA_PERIODIC_WRAP) ? 2 * GW : 0);
-        TOSCA_LAUNCH("k_wrap_axis", k_wrap_axis<T>, dim3((n1 + 127) / 128, n2, 2 * GW), dim3(128), 0, s, a, ncomp, g, axis);
+    int olo[3], ohi[3], clo[3], chi[3];
+    for (int q = 0; q < 3; q++) {
+        const bool per = g.per[q] != TOSCA_PERIODIC_NONE, wrap = g.per[q] == TOSCA_PERIODIC_WRAP;
+        olo[q] = wrap ? -GW : 0; ohi[q] = wrap ? m[q] + GW : m[q];
+        clo[q] = per && reset != RESET_NONE ? 1 : 0; chi[q] = per && reset == RESET_CELL ? m[q] - 1 : m[q];
     }
+    return make_shell(olo, ohi, clo, chi);
 }
+template <class T>
+void ghosts(T *a, int ncomp, const Geo &g, int reset, hipStream_t s) {
+    const Shell B = ghost_shell(g, reset);
+    if (B.total) TOSCA_LAUNCH("k_ghosts", k_ghosts<T>, dim3((B.total + 255) / 256), dim3(256), 0, s, a, ncomp, g, B, reset);
+}
+}  // namespace
+
+template <class T>
+void launch_wrap(T *a, int ncomp, const Geo &g, hipStream_t s) { ghosts(a, ncomp, g, RESET_NONE, s); }
 template void launch_wrap<double>(double *, int, const Geo &, hipStream_t);
 template void launch_wrap<float>(float *, int, const Geo &, hipStream_t);
 
-void launch_reset_cell_periodic(double *a, int ncomp, const Geo &g, hipStream_t s) {
-    const int m[3] = {g.mx, g.my, g.mz};
-    for (int axis = 0; axis < 3; axis++) {
-        if (g.per[axis] == TOSCA_PERIODIC_NONE) continue;
-        int t1 = (axis == 0) ? 1 : 0, t2 = (axis == 2) ? 1 : 2;
-        TOSCA_LAUNCH("k_reset_axis", k_reset_axis, dim3((m[t1] + 127) / 128, m[t2], 2), dim3(128), 0, s, a, ncomp, g, axis);
-    }
-    launch_wrap(a, ncomp, g, s);
-}
-
-// resetFacePeriodicFluxesVector (src/include/inline.h:5357-5451): on each periodic axis the
-// points of index 0 take the values at m-2 (type 1; type 2 reads ghost -2, which holds m-2),
-// then the ghost scatter; the side-0 launch of k_reset_axis
-void launch_reset_face_periodic(double *a, int ncomp, const Geo &g, hipStream_t s) {
-    const int m[3] = {g.mx, g.my, g.mz};
-    for (int axis = 0; axis < 3; axis++) {
-        if (g.per[axis] == TOSCA_PERIODIC_NONE) continue;
-        int t1 = (axis == 0) ? 1 : 0, t2 = (axis == 2) ? 1 : 2;
-        TOSCA_LAUNCH("k_reset_axis", k_reset_axis, dim3((m[t1] + 127) / 128, m[t2], 1), dim3(128), 0, s, a, ncomp, g, axis);
-    }
-    launch_wrap(a, ncomp, g, s);
-}
+void launch_reset_cell_periodic(double *a, int ncomp, const Geo &g, hipStream_t s) { ghosts(a, ncomp, g, RESET_CELL, s); }
+void launch_reset_face_periodic(double *a, int ncomp, const Geo &g, hipStream_t s) { ghosts(a, ncomp, g, RESET_FACE, s); }
 
 void launch_fill(double *a, long n, double v, hipStream_t s) {
     TOSCA_LAUNCH("k_fill", k_fill, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a, n, v);
@@ -568,34 +562,32 @@ void ref_update_cs(const Geo &g, const tosca_mesh *m, const tosca_params *p, con
                      part, g);
         TOSCA_LAUNCH("k_dpasd_cs", k_dpasd_cs, gi, blk2(), 0, s, part, cs, p->max_cs, g);
     }
-    launch_wrap(cs, 1, g, s);
-    launch_reset_cell_periodic(cs, 1, g, s);
+    launch_reset_cell_periodic(cs, 1, g, s);           // (and the wraps)
 }
 
 void ref_update_nut(const Geo &g, const tosca_mesh *m, const tosca_params *p, const double *ucat, const double *cs,
                     double *nut, double *ksgs, hipStream_t s) {
     const long n = g.nloc();
-    launch_fill(nut, n, 0.0, s);
-    if (ksgs) launch_fill(ksgs, n, 0.0, s);
     TOSCA_LAUNCH("k_nut", k_nut, grd(g.mx - 2, g.my - 2, g.mz - 2), blk2(), 0, s, ucat, m->csi, m->eta, m->zet, m->aj,
                        cs, nut, ksgs, g);
-    launch_nut_bcs(nut, p, g, s);
-    if (ksgs) launch_wrap(ksgs, 1, g, s);
+    launch_nut_ghosts(nut, p, g, s);
+    if (ksgs) launch_nut_ghosts(ksgs, static_cast<const tosca_params *>(nullptr), g, s);
 }
 
 template <class T>
-void launch_nut_bcs(T *nut, const tosca_params *p, const Geo &g, hipStream_t s) {
+void launch_nut_ghosts(T *nut, const tosca_params *p, const Geo &g, hipStream_t s, double *cs, double cs_fill) {
     NutBC B;
-    for (int q = 0; q < 6; q++) { B.bc[q] = p->bc_nut[q]; B.val[q] = p->nut_value[q]; }
-    const int mm[3] = {g.mx, g.my, g.mz};
-    for (int axis = 0; axis < 3; axis++) {
-        int t1 = (axis == 0) ? 1 : 0, t2 = (axis == 2) ? 1 : 2;
-        TOSCA_LAUNCH("k_nut_bc", k_nut_bc<T>, dim3((mm[t1] + 127) / 128, mm[t2] - 2, 2), dim3(128), 0, s, nut, B, g, axis);
-    }
-    launch_wrap(nut, 1, g, s);
+    for (int q = 0; q < 6; q++) { B.bc[q] = p ? p->bc_nut[q] : -1; B.val[q] = p ? p->nut_value[q] : 0.0; }
+    const int olo[3] = {-GW, -GW, -GW}, ohi[3] = {g.mx + GW, g.my + GW, g.mz + GW}, clo[3] = {1, 1, 1},
+              chi[3] = {g.mx - 1, g.my - 1, g.mz - 1};
+    const Shell S = make_shell(olo, ohi, clo, chi);
+    Shell C{};
+    if (cs && cs_fill < 0.0) C = ghost_shell(g, RESET_CELL);
+    TOSCA_LAUNCH("k_nut_ghosts", k_nut_ghosts<T>, dim3((S.total + C.total + 255) / 256), dim3(256), 0, s, nut, B, g, S, cs,
+                 cs ? cs_fill : -1.0, C);
 }
-template void launch_nut_bcs<double>(double *, const tosca_params *, const Geo &, hipStream_t);
-template void launch_nut_bcs<float>(float *, const tosca_params *, const Geo &, hipStream_t);
+template void launch_nut_ghosts<double>(double *, const tosca_params *, const Geo &, hipStream_t, double *, double);
+template void launch_nut_ghosts<float>(float *, const tosca_params *, const Geo &, hipStream_t, double *, double);
 
 void ref_buoyancy(const Geo &g, const tosca_mesh *m, const tosca_params *p, const double *theta, double scale,
                   double *btheta, double *gcont, hipStream_t s) {

@@ -772,8 +772,7 @@ void vjp_rhs_impl(const Geo &g, const tosca_mesh *mesh, const tosca_params *p, c
     const dim3 cb(64, 4), cg((g.mx - 2 + 63) / 64, (g.my - 2 + 3) / 4, g.mz - 2);
     if (renut) {
         TOSCA_LAUNCH(f32 ? "k_vjp_pre_f32" : "k_vjp_pre", (k_vjp_pre<T, P>), cg, cb, 0, s, A, g);
-        zero_outside_interior(nut, g, s);
-        nut_bcs(nut, p, g, s);
+        launch_nut_ghosts(nut, p, g, s);
     } else {
         TOSCA_LAUNCH(f32 ? "k_vjp_fp_f32" : "k_vjp_fp", (k_vjp_fp<T, P>), cg, cb, 0, s, A, g);
     }
