@@ -134,36 +134,85 @@ __device__ __forceinline__ FluxT<T> face_general(const FormUArgsT<T, MT> &A, con
     return face_flux<2>(A, g, a, b, f);
 }
 
-template <class T, class MT>
-__global__ void __launch_bounds__(128) k_formu_boundary(FormUArgsT<T, MT> A, Geo g, BoundaryBufs B) {
-    const int d = blockIdx.z / 3, what = blockIdx.z % 3;      // what: 0 face 0, 1 face m-2, 2 seam fp
+// One launch of workgroups of six waves.  Those of the boundary faces take 384 positions of a direction's
+// two faces (of a periodic axis, whose face 0 is face m-2, of the one); those of a seam take 64 cells, one
+// of their six faces a wave, and add the fluxes through LDS: a face is a chain of loads, which a thread that
+// took all six waited for six times.  Across i every point is a cache line of its own, so a wave takes 8 x 8
+// positions, whose 100 rows fit in L1; 64 of one row j with their neighbours do not.
+// Bound by the latency of those chains and by the lines across i, which take three quarters of the launch at
+// 512 x 512 x 192.  Against one face or one whole seam cell a thread, 64 along a row: 22 -> 16 us at 64^3 with
+// three seams, 16 -> 9 at 16 x 10 x 8, 53 -> 44 at 256 x 128 x 96, 248 -> 174 at 512 x 512 x 192.
+struct BoundaryGrid { int face0[3], seam0[3], total; };    // first workgroup of each list, in the order d0 faces, d0 seam, d1 ...
+constexpr int FB_THREADS = 384;
+// positions of direction d, with those of the i faces padded to whole 8 x 8 tiles
+__host__ __device__ inline int boundary_positions(const Geo &g, int d) {
     int n1, n2;
     const int n = tr_dims(g, d, n1, n2);
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const int a = t % n1, b = t / n1;
-    const int ma = (d == 0) ? g.my : g.mx, mb = (d == 2) ? g.my : g.mz;
-    if (a < 1 || a > ma - 2 || b < 1 || b > mb - 2) return;     // transverse interior only
+    return d == 0 ? ((n1 + 7) / 8) * ((n2 + 7) / 8) * 64 : n;
+}
+inline BoundaryGrid boundary_grid(const Geo &g) {
+    BoundaryGrid G;
+    int b = 0;
+    for (int d = 0; d < 3; d++) {
+        const int n = boundary_positions(g, d);
+        const bool per = g.per[d] != TOSCA_PERIODIC_NONE;
+        G.face0[d] = b; b += ((per ? n : 2 * n) + FB_THREADS - 1) / FB_THREADS;
+        G.seam0[d] = b; b += per ? (n + 63) / 64 : 0;
+    }
+    G.total = b;
+    return G;
+}
+
+template <class T, class MT>
+__global__ void __launch_bounds__(FB_THREADS) k_formu_boundary(FormUArgsT<T, MT> A, Geo g, BoundaryBufs B, BoundaryGrid G) {
+    __shared__ T sF[6][6][64];
+    const int blk = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int d = blk >= G.face0[2] ? 2 : blk >= G.face0[1] ? 1 : 0;
+    const int seam0 = d == 0 ? G.seam0[0] : d == 1 ? G.seam0[1] : G.seam0[2], face0 = d == 0 ? G.face0[0] : d == 1 ? G.face0[1] : G.face0[2];
+    const bool seam = blk >= seam0;
+    const bool per = (d == 0 ? g.per[0] : d == 1 ? g.per[1] : g.per[2]) != TOSCA_PERIODIC_NONE;
+    int n1, n2;
+    const int n = tr_dims(g, d, n1, n2), np = boundary_positions(g, d);
+    const int p = seam ? (blk - seam0) * 64 + lane : (blk - face0) * FB_THREADS + (int)threadIdx.x;
+    const int what = per || p >= np ? 1 : 0, q = !seam && !per && what ? p - np : p;            // 0 face 0, 1 face m-2
+    int a = q % n1, b = q / n1;
+    if (d == 0) {
+        const int tile = q / 64, tj = (n1 + 7) / 8;
+        a = tile % tj * 8 + (q & 7);
+        b = tile / tj * 8 + ((q >> 3) & 7);
+    }
+    const int t = b * n1 + a;
+    const bool on = q < np && a >= 1 && a <= n1 - 2 && b >= 1 && b <= n2 - 2;                   // transverse interior only
     const int m = (d == 0) ? g.mx : (d == 1) ? g.my : g.mz;
-    if (what < 2) {
-        const int f = what == 0 ? 0 : m - 2;
-        FluxT<T> F = (d == 0) ? face_general<0>(A, g, f, a, b) : (d == 1) ? face_general<1>(A, g, f, a, b)
-                                                                        : face_general<2>(A, g, f, a, b);
-        double *o = B.bF[d] + ((long)what * n + t) * 6;
-        o[0] = F.d.x; o[1] = F.d.y; o[2] = F.d.z; o[3] = F.v.x; o[4] = F.v.y; o[5] = F.v.z;
+    // the face: dir at index f, transverse (u, v); of a seam cell (index 1 along d) the upper or lower face
+    // of direction w / 2
+    int x[3], dir = d, f = what ? m - 2 : 0, u = a, v = b;
+    if (seam) {
+        x[0] = d == 0 ? 1 : a; x[1] = d == 1 ? 1 : d == 0 ? a : b; x[2] = d == 2 ? 1 : b;
+        dir = w >> 1;
+        f = (dir == 0 ? x[0] : dir == 1 ? x[1] : x[2]) - (w & 1);
+        u = dir == 0 ? x[1] : x[0];
+        v = dir == 2 ? x[1] : x[2];
+    }
+    dir = __builtin_amdgcn_readfirstlane(dir);
+    FluxT<T> F{{0, 0, 0}, {0, 0, 0}};
+    if (on) F = dir == 0 ? face_general<0>(A, g, f, u, v) : dir == 1 ? face_general<1>(A, g, f, u, v) : face_general<2>(A, g, f, u, v);
+    if (!seam) {
+        if (!on) return;
+        for (int e = per ? 0 : what; e <= what; e++) {
+            double *o = (d == 0 ? B.bF[0] : d == 1 ? B.bF[1] : B.bF[2]) + ((long)e * n + t) * 6;
+            o[0] = F.d.x; o[1] = F.d.y; o[2] = F.d.z; o[3] = F.v.x; o[4] = F.v.y; o[5] = F.v.z;
+        }
         return;
     }
-    if (g.per[d] == TOSCA_PERIODIC_NONE) return;
-    // fp at cell 1 along d (transverse interior), from its six faces
-    int i, j, k;
-    if (d == 0) { i = 1; j = a; k = b; } else if (d == 1) { i = a; j = 1; k = b; } else { i = a; j = b; k = 1; }
-    const FluxT<T> f1 = face_general<0>(A, g, i, j, k), f1m = face_general<0>(A, g, i - 1, j, k);
-    const FluxT<T> f2 = face_general<1>(A, g, j, i, k), f2m = face_general<1>(A, g, j - 1, i, k);
-    const FluxT<T> f3 = face_general<2>(A, g, k, i, j), f3m = face_general<2>(A, g, k - 1, i, j);
-    double *o = B.seam[d] + (long)t * 3;
-    o[0] = fpsum(f1.d.x, f1m.d.x, f2.d.x, f2m.d.x, f3.d.x, f3m.d.x, f1.v.x, f1m.v.x, f2.v.x, f2m.v.x, f3.v.x, f3m.v.x, A.mode);
-    o[1] = fpsum(f1.d.y, f1m.d.y, f2.d.y, f2m.d.y, f3.d.y, f3m.d.y, f1.v.y, f1m.v.y, f2.v.y, f2m.v.y, f3.v.y, f3m.v.y, A.mode);
-    o[2] = fpsum(f1.d.z, f1m.d.z, f2.d.z, f2m.d.z, f3.d.z, f3m.d.z, f1.v.z, f1m.v.z, f2.v.z, f2m.v.z, f3.v.z, f3m.v.z, A.mode);
+    sF[w][0][lane] = F.d.x; sF[w][1][lane] = F.d.y; sF[w][2][lane] = F.d.z;
+    sF[w][3][lane] = F.v.x; sF[w][4][lane] = F.v.y; sF[w][5][lane] = F.v.z;
+    __syncthreads();
+    if (w >= 3 || !on) return;
+    // fp at the cell, component w
+    (d == 0 ? B.seam[0] : d == 1 ? B.seam[1] : B.seam[2])[(long)t * 3 + w] =
+        fpsum(sF[0][w][lane], sF[1][w][lane], sF[2][w][lane], sF[3][w][lane], sF[4][w][lane], sF[5][w][lane], sF[0][3 + w][lane],
+              sF[1][3 + w][lane], sF[2][3 + w][lane], sF[3][3 + w][lane], sF[4][3 + w][lane], sF[5][3 + w][lane], A.mode);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -643,8 +692,8 @@ void fused_formu(const Geo &g, const FormUArgsT<T, MT> &A, double *ws, hipStream
     for (int d = 0; d < 3; d++) { const long n = tr_dims(g, d, n1, n2); B.seam[d] = ws + off; off += n * 3; }
     const int nsj = (g.my - 2 + TJ - 1) / TJ;                 // j tiles; the last one has no seam
     double *sv1 = ws + off, *sv2 = ws + off + (long)nsj * g.mz * g.mx;
-    const int nmax = max(g.my * g.mz, max(g.mx * g.mz, g.mx * g.my));
-    TOSCA_LAUNCH(sizeof(T) == 8 ? "k_formu_boundary" : sizeof(MT) == 8 ? "k_formu_boundary_f32" : "k_formu_boundary_f32m", (k_formu_boundary<T, MT>), dim3((nmax + 127) / 128, 1, 9), dim3(128), 0, s, A, g, B);
+    const BoundaryGrid G = boundary_grid(g);
+    TOSCA_LAUNCH(sizeof(T) == 8 ? "k_formu_boundary" : sizeof(MT) == 8 ? "k_formu_boundary_f32" : "k_formu_boundary_f32m", (k_formu_boundary<T, MT>), dim3(G.total), dim3(FB_THREADS), 0, s, A, g, B, G);
 
     MainArgs<T, MT> M;
     // the main kernel loads nu_t unconditionally; without LES (or without the viscous term) the
