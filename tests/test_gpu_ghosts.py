@@ -82,3 +82,25 @@ def test_predictor_ghosts(n, periodic):
     for name, a, b in zip(("ucont", "ucat", "rhs", "utmp"), g, (uc, ua, rhs, utmp)):
         assert relerr(to_np(a), b) <= TOL, name
     ctx.close()
+
+
+@pytest.mark.parametrize("periodic", PERS)
+@pytest.mark.parametrize("n", SIZES)
+def test_predictor_ghosts_transposed(n, periodic):
+    """<xbar, J d> = <J^T xbar, d> of two RK3W stages against the tangent oracle: the transposed copies of
+    the smallest axes, on which every point has several.  About 100 roundings a product against the sum of
+    the sizes of at most 1e4 terms, with a wrong value among them showing as 1e-4: bound 1e-10."""
+    lay, nm, dm, f, po, pg, ctx, keep = _setup(n, periodic, 9, C.LES_DSM)
+    rng = np.random.default_rng(10)
+    shape = (lay.mz, lay.my, lay.mx, 3)
+    dp, bt, xbar, du = (rng.standard_normal(shape) for _ in range(4))
+    dn, dt = rng.standard_normal(lay.gshape), 0.02
+    work = [torch.zeros(shape, dtype=torch.float64, device="cuda") for _ in range(3)]
+    ub, nb = to_dev(xbar), torch.zeros(lay.gshape, dtype=torch.float64, device="cuda")
+    ctx.UeqnRK3W_adjoint(dm, pg, to_dev(f["ucont"]), to_dev(f["ucat"]), to_dev(f["nut"]), to_dev(dp), to_dev(bt), None, 0, None,
+                         dt, 2, *work, ub, nb)
+    for d, bar in ((dict(d_ucont=du), np.sum(to_np(ub) * du)), (dict(d_nut=dn), np.sum(to_np(nb) * dn))):
+        _, dF = O.rk3w_jvp(lay.info(), nm, po, f["ucont"], f["ucat"], f["nut"], dp, bt, None, 0, None, dt, 2, **d)
+        err = abs(np.sum(xbar * dF) - bar) / (np.sum(np.abs(xbar * dF)) + 1e-300)
+        assert err <= 1e-10, (d.keys(), err)
+    ctx.close()

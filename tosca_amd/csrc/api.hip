@@ -418,10 +418,8 @@ void queue_explicit(tosca_ctx *c, const tosca_mesh *m, const tosca_params *p, do
     const Geo &g = c->geo;
     hipStream_t s = c->stream;
     const bool visc = form_mode != 1;
-    tosca::launch_no_penetration(ucont, p, g, s);                    // ueqn_solvers.c:1281
-    tosca::launch_reset_face_periodic(ucont, 3, g, s);               // :1284
-    tosca::launch_contra_to_cart(ucont, m, ucat, g, s);              // :1287
-    tosca::launch_reset_cell_periodic(ucat, 3, g, s);                // :1301
+    tosca::launch_face_resets(ucont, p, g, s);                       // ueqn_solvers.c:1281-1284
+    tosca::launch_contra_to_cart(ucont, m, ucat, g, s);              // :1287-1301
     tosca::launch_rhs_init(rhs, dp, btheta, ab2 ? btheta_o : nullptr, btheta ? ab2 : 0, farm, g, s);   // :1304-1344
     const double *nu_t = (p->les_active && visc) ? nut : nullptr;   // :1347
     if (c->ref_path) {
@@ -440,10 +438,8 @@ void queue_imex(tosca_ctx *c, const tosca_mesh *m, const tosca_params *p, const 
     hipStream_t s = c->stream;
     const long ng3 = 3L * g.mx * g.my * g.mz;
     tosca::launch_global_to_local(ucont, v, g, s);                         // :1763-1767 (wrapped below)
-    tosca::launch_no_penetration(ucont, p, g, s);                          // :1770
-    tosca::launch_reset_face_periodic(ucont, 3, g, s);                     // :1773
-    tosca::launch_contra_to_cart(ucont, m, ucat, g, s);                    // :1777
-    tosca::launch_reset_cell_periodic(ucat, 3, g, s);                      // :1790
+    tosca::launch_face_resets(ucont, p, g, s);                             // :1770-1773
+    tosca::launch_contra_to_cart(ucont, m, ucat, g, s);                    // :1777-1790
     tosca::launch_fill(av, ng3, 0.0, s);                                   // :1793
     const double *nu_t = p->les_active ? nut : nullptr;
     if (c->ref_path) {                                                     // :1794
@@ -997,29 +993,24 @@ int tosca_ueqn_rk3w_adjoint(tosca_ctx *c, const tosca_mesh *m, const tosca_param
         const double *x = chk + (size_t)st * ng3, *uo = chk + (size_t)(st - i) * ng3;
         // the stage's reset fluxes and Cartesian velocity, recomputed from its checkpoint
         tosca::launch_global_to_local(ucont, x, g, s);
-        tosca::launch_no_penetration(ucont, p, g, s);
-        tosca::launch_reset_face_periodic(ucont, 3, g, s);
+        tosca::launch_face_resets(ucont, p, g, s);
         tosca::launch_contra_to_cart(ucont, m, ucat, g, s);
-        tosca::launch_reset_cell_periodic(ucat, 3, g, s);
         // cotangent of the stage's Rhs; resetNonResolvedCellFaces zeroes the same entries of it
         tosca::launch_rk3w_adj_combine(ucont_bar, carry, rbar, dt * kWrayBeta[i], -1.0 * dt * kWrayDelta[i], g, s);
         tosca::launch_non_resolved(rbar, uo, p, g, s);
         // FormU (the sources are constant): cotangents of the local ucont, ucat and nu_t
         tosca::vjp_formu_nut(g, m, p, ucont, ucat, nut, rbar, 1.0, vbar, ubar, les ? nut_bar : nullptr, c->ws, s);
         // contravariantToCartesian and the periodic resets of ucat, transposed into the ucont cotangent
-        tosca::launch_reset_cell_periodic_adj(ubar, 3, g, s);
-        tosca::launch_c2c_adj(ubar, m, qbar, vbar, g, s);
+        tosca::launch_reset_cell_periodic_adj(ubar, g, s);
         // the stage update reads the reset state: its cotangent is the next state's plus ExplicitRhsU's
-        tosca::launch_add_owned(ucont_bar, vbar, g, s);
+        tosca::launch_c2c_adj(ubar, m, qbar, vbar, ucont_bar, g, s);
         tosca::launch_face_resets_adj(ucont_bar, x, p, g, s);
     }
     // leave ucont and ucat as the forward sweep left them
     if (n_stages > 0) {
         tosca::launch_global_to_local(ucont, chk + (size_t)(n_stages - 1) * ng3, g, s);
-        tosca::launch_no_penetration(ucont, p, g, s);
-        tosca::launch_reset_face_periodic(ucont, 3, g, s);
+        tosca::launch_face_resets(ucont, p, g, s);
         tosca::launch_contra_to_cart(ucont, m, ucat, g, s);
-        tosca::launch_reset_cell_periodic(ucat, 3, g, s);
         tosca::launch_global_to_local(ucont, chk + (size_t)n_stages * ng3, g, s);
         tosca::launch_wrap(ucont, 3, g, s);
     }
@@ -1211,10 +1202,8 @@ int tosca_snes_func_eval(tosca_ctx *c, const tosca_mesh *m, const tosca_params *
     if (F == u || F == bU || F == ucont_o) return set_err(c, TOSCA_ERR_ARG, "F must not alias an input");
     hipStream_t s = c->stream;
     tosca::launch_global_to_local(ucont, u, g, s);                           // :1195-1199 (wrapped below)
-    tosca::launch_no_penetration(ucont, p, g, s);                            // :1202
-    tosca::launch_reset_face_periodic(ucont, 3, g, s);                       // :1205
-    tosca::launch_contra_to_cart(ucont, m, ucat, g, s);                      // :1208
-    tosca::launch_reset_cell_periodic(ucat, 3, g, s);                        // :1221
+    tosca::launch_face_resets(ucont, p, g, s);                               // :1202-1205
+    tosca::launch_contra_to_cart(ucont, m, ucat, g, s);                      // :1208-1221
     if (hipMemcpyAsync(F, bU, vb, hipMemcpyDeviceToDevice, s) != hipSuccess)  // :1224
         return set_err(c, TOSCA_ERR_DEVICE, "SNESFuncEval: copy failed");
     const double scale = ab2 ? 0.5 : 1.0;                                     // :1227

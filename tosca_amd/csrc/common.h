@@ -454,13 +454,48 @@ inline Shell make_shell(const int (&olo)[3], const int (&ohi)[3], const int (&cl
 }
 __device__ __forceinline__ bool shell_point(const Shell &B, int t, int &i, int &j, int &k) {
     if (t >= B.total) return false;
-    int q = 0, start = 0;
-    while (t >= B.end[q]) start = B.end[q++];
-    const int e = t - start, r = e / B.ni[q];
-    i = B.i0[q] + e % B.ni[q];
-    j = B.j0[q] + r % B.nj[q];
-    k = B.k0[q] + r / B.nj[q];
+    int start = 0, i0 = B.i0[0], j0 = B.j0[0], k0 = B.k0[0], ni = B.ni[0], nj = B.nj[0];
+#pragma unroll
+    for (int q = 1; q < 6; q++) {               // (constant indices: a runtime one puts B in scratch memory)
+        const bool in = t >= B.end[q - 1];
+        start = in ? B.end[q - 1] : start;
+        i0 = in ? B.i0[q] : i0; j0 = in ? B.j0[q] : j0; k0 = in ? B.k0[q] : k0;
+        ni = in ? B.ni[q] : ni; nj = in ? B.nj[q] : nj;
+    }
+    const int e = t - start, r = e / ni;
+    i = i0 + e % ni;
+    j = j0 + r % nj;
+    k = k0 + r / nj;
     return true;
 }
 
+// DMLocalToLocal on the DM_BOUNDARY_PERIODIC axes (ghost layers take the wrapped owned values; the other
+// axes keep their ghosts), after the periodic resets of `reset` (src/include/inline.h):
+//   RESET_CELL  resetCellPeriodicFluxes (:5496-5514): the boundary cells 0 / m-1 of a periodic axis take
+//               cells m-2 / 1 over the whole owned range of the other two axes
+//   RESET_FACE  resetFacePeriodicFluxesVector (:5357-5451): the points of index 0 take the values at m-2
+//               (type 1; type 2 reads ghost -2, which holds m-2)
+// one axis after the other.  A written point's source is no written point, so the axes compose.
+enum { RESET_NONE, RESET_FACE, RESET_CELL };
+__device__ __forceinline__ int ghost_source(int x, int m, int per, int reset) {
+    if (per == TOSCA_PERIODIC_NONE) return x;
+    if (per == TOSCA_PERIODIC_WRAP) x = x < 0 ? x + m : x >= m ? x - m : x;
+    if (reset != RESET_NONE && x == 0) return m - 2;
+    if (reset == RESET_CELL && x == m - 1) return 1;
+    return x;
+}
+__device__ __forceinline__ int ghost_point(const Geo &g, int i, int j, int k, int reset) {
+    return g.L(ghost_source(k, g.mz, g.per[2], reset), ghost_source(j, g.my, g.per[1], reset), ghost_source(i, g.mx, g.per[0], reset));
+}
+// the points written
+inline Shell ghost_shell(const Geo &g, int reset) {
+    const int m[3] = {g.mx, g.my, g.mz};
+    int olo[3], ohi[3], clo[3], chi[3];
+    for (int q = 0; q < 3; q++) {
+        const bool per = g.per[q] != TOSCA_PERIODIC_NONE, wrap = g.per[q] == TOSCA_PERIODIC_WRAP;
+        olo[q] = wrap ? -GW : 0; ohi[q] = wrap ? m[q] + GW : m[q];
+        clo[q] = per && reset != RESET_NONE ? 1 : 0; chi[q] = per && reset == RESET_CELL ? m[q] - 1 : m[q];
+    }
+    return make_shell(olo, ohi, clo, chi);
+}
 }  // namespace tosca

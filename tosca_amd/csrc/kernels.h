@@ -10,7 +10,6 @@ namespace tosca {
 // resetCellPeriodicFluxes, after resetFacePeriodicFluxesVector; and nu_t outside the interior cells
 template <class T> void launch_wrap(T *a, int ncomp, const Geo &g, hipStream_t s);
 void launch_reset_cell_periodic(double *a, int ncomp, const Geo &g, hipStream_t s);
-void launch_reset_face_periodic(double *a, int ncomp, const Geo &g, hipStream_t s);
 void launch_fill(double *a, long n, double v, hipStream_t s);
 // (p null: no patch kinds, as for a scalar that is zero there); cs given: in the same launch Cs outside the
 // interior, the constant cs_fill or (< 0) its periodic resets and wraps
@@ -27,8 +26,17 @@ void ref_update_nut(const Geo &g, const tosca_mesh *m, const tosca_params *p, co
 void ref_buoyancy(const Geo &g, const tosca_mesh *m, const tosca_params *p, const double *theta, double scale,
                   double *btheta, double *gcont, hipStream_t s);
 
+// boundaryU kinds of the patches: iLeft iRight jLeft jRight kLeft kRight
+struct PatchKinds { int bc[6]; };
+inline PatchKinds patch_kinds(const tosca_params *p) {
+    PatchKinds P;
+    for (int q = 0; q < 6; q++) P.bc[q] = p->bc_u[q];
+    return P;
+}
+
 // ExplicitRhsU steps around FormU (explicit_rhs.hip)
-void launch_no_penetration(double *ucont, const tosca_params *p, const Geo &g, hipStream_t s);
+// (the no-penetration and the periodic face resets of ucont, with its wraps; ucat with its periodic resets and wraps)
+void launch_face_resets(double *ucont, const tosca_params *p, const Geo &g, hipStream_t s);
 void launch_contra_to_cart(const double *ucont, const tosca_mesh *m, double *ucat, const Geo &g, hipStream_t s);
 void launch_rhs_init(double *rhs, const double *dp, const double *bt, const double *bto, int ab2, const double *farm,
                      const Geo &g, hipStream_t s);
@@ -49,9 +57,9 @@ void launch_rk3w_update(double *ucont, const double *rhs, double *rhs_o, double 
                         hipStream_t s);
 void launch_rk3w_adj_combine(const double *xbar, double *carry, double *rbar, double a, double b, const Geo &g,
                              hipStream_t s);
-void launch_reset_cell_periodic_adj(double *a, int ncomp, const Geo &g, hipStream_t s);
-void launch_c2c_adj(const double *ubar, const tosca_mesh *m, double *qbar, double *vbar, const Geo &g, hipStream_t s);
-void launch_add_owned(double *xbar, const double *vbar, const Geo &g, hipStream_t s);
+void launch_reset_cell_periodic_adj(double *a, const Geo &g, hipStream_t s);
+void launch_c2c_adj(const double *ubar, const tosca_mesh *m, double *qbar, const double *vbar, double *xbar, const Geo &g,
+                    hipStream_t s);
 void launch_face_resets_adj(double *xbar, const double *x, const tosca_params *p, const Geo &g, hipStream_t s);
 
 // Krylov vector kernels (krylov.hip)

@@ -17,24 +17,6 @@ namespace tosca {
 // ---------------------------------------------------------------------------------------------
 // ghost handling
 // ---------------------------------------------------------------------------------------------
-// DMLocalToLocal on the DM_BOUNDARY_PERIODIC axes (ghost layers take the wrapped owned values; the other
-// axes keep their ghosts), after the periodic resets of `reset` (src/include/inline.h):
-//   RESET_CELL  resetCellPeriodicFluxes (:5496-5514): the boundary cells 0 / m-1 of a periodic axis take
-//               cells m-2 / 1 over the whole owned range of the other two axes
-//   RESET_FACE  resetFacePeriodicFluxesVector (:5357-5451): the points of index 0 take the values at m-2
-//               (type 1; type 2 reads ghost -2, which holds m-2)
-// one axis after the other.  A written point's source is no written point, so the axes compose.
-enum { RESET_NONE, RESET_FACE, RESET_CELL };
-__device__ __forceinline__ int ghost_source(int x, int m, int per, int reset) {
-    if (per == TOSCA_PERIODIC_NONE) return x;
-    if (per == TOSCA_PERIODIC_WRAP) x = x < 0 ? x + m : x >= m ? x - m : x;
-    if (reset != RESET_NONE && x == 0) return m - 2;
-    if (reset == RESET_CELL && x == m - 1) return 1;
-    return x;
-}
-__device__ __forceinline__ int ghost_point(const Geo &g, int i, int j, int k, int reset) {
-    return g.L(ghost_source(k, g.mz, g.per[2], reset), ghost_source(j, g.my, g.per[1], reset), ghost_source(i, g.mx, g.per[0], reset));
-}
 template <class T>
 __global__ void __launch_bounds__(256) k_ghosts(T *a, int ncomp, Geo g, Shell B, int reset) {
     int i, j, k;
@@ -490,17 +472,6 @@ static inline dim3 blk2() { return dim3(64, 4, 1); }
 static inline dim3 grd(int ni, int nj, int nk) { return dim3((ni + 63) / 64, (nj + 3) / 4, nk); }
 
 namespace {
-// the points k_ghosts writes
-Shell ghost_shell(const Geo &g, int reset) {
-    const int m[3] = {g.mx, g.my, g.mz};
-    int olo[3], ohi[3], clo[3], chi[3];
-    for (int q = 0; q < 3; q++) {
-        const bool per = g.per[q] != TOSCA_PERIODIC_NONE, wrap = g.per[q] == TOSCA_PERIODIC_WRAP;
-        olo[q] = wrap ? -GW : 0; ohi[q] = wrap ? m[q] + GW : m[q];
-        clo[q] = per && reset != RESET_NONE ? 1 : 0; chi[q] = per && reset == RESET_CELL ? m[q] - 1 : m[q];
-    }
-    return make_shell(olo, ohi, clo, chi);
-}
 template <class T>
 void ghosts(T *a, int ncomp, const Geo &g, int reset, hipStream_t s) {
     const Shell B = ghost_shell(g, reset);
@@ -514,7 +485,6 @@ template void launch_wrap<double>(double *, int, const Geo &, hipStream_t);
 template void launch_wrap<float>(float *, int, const Geo &, hipStream_t);
 
 void launch_reset_cell_periodic(double *a, int ncomp, const Geo &g, hipStream_t s) { ghosts(a, ncomp, g, RESET_CELL, s); }
-void launch_reset_face_periodic(double *a, int ncomp, const Geo &g, hipStream_t s) { ghosts(a, ncomp, g, RESET_FACE, s); }
 
 void launch_fill(double *a, long n, double v, hipStream_t s) {
     TOSCA_LAUNCH("k_fill", k_fill, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a, n, v);

@@ -8,21 +8,19 @@
 //                        range of the local ucont, and Rhs_o = Rhs (:1533-1541, :1563-1569)
 // Adjoint (the transpose of each forward step, in reverse order; no reference counterpart):
 //   k_rk3w_adj_combine   cotangent of the stage's Rhs from the two stage updates that read it
-//   k_reset_axis_adj     transpose of resetCellPeriodicFluxes' boundary copies (inline.h:5496-5514)
-//   k_wrap_axis_adj      transpose of the periodic ghost scatter (DMLocalToLocal)
+//   k_ghosts_adj         transpose of resetCellPeriodicFluxes' boundary copies (inline.h:5496-5514) and of the
+//                        periodic ghost scatter (DMLocalToLocal)
 //   k_c2c_adj_solve      transpose of contravariantToCartesian's 3x3 solve (src/ueqn.c:571-613)
-//   k_c2c_adj_gather     transpose of its face averages (inline.h:4307-4310), added to ucont_bar
-//   k_add_owned          the owned range of a local cotangent added to a global one
-//   k_face_periodic_adj  transpose of resetFacePeriodicFluxesVector's face-0 copy (inline.h:5357-5451)
-//   k_no_penetration_adj transpose of resetNoPenetrationFluxes (inline.h:5262-5355): the zeroed
-//                        fluxes carry no cotangent; a zeroGradient flux only where it was not clipped
+//   k_c2c_adj_gather     transpose of its face averages (inline.h:4307-4310), added with FormU's ucont
+//                        cotangent to the global one
+//   k_face_resets_adj    transpose of resetFacePeriodicFluxesVector's face-0 copies (inline.h:5357-5451), then
+//                        of resetNoPenetrationFluxes (inline.h:5262-5355): the zeroed fluxes carry no
+//                        cotangent; a zeroGradient flux only where it was not clipped
 #include "kernels.h"
 
 namespace tosca {
 
 namespace {
-
-struct Kinds { int bc[6]; };
 
 __device__ __forceinline__ long owned_local(const Geo &g, long q) {
     const int i = (int)(q % g.mx);
@@ -57,54 +55,40 @@ __global__ void k_rk3w_adj_combine(const double *xbar, double *carry, double *rb
     carry[t] = b * x;
 }
 
-// transpose of a copy a[dst] = a[src]: abar[src] += abar[dst]; abar[dst] = 0.  Within one launch
-// the destinations are distinct, the sources are distinct and no source is a destination, so the
-// threads touch disjoint points.
-__device__ __forceinline__ void copy_adj(double *a, int ncomp, long cd, long cs) {
-    for (int q = 0; q < ncomp; q++) {
-        a[ncomp * cs + q] = a[ncomp * cs + q] + a[ncomp * cd + q];
-        a[ncomp * cd + q] = 0.0;
-    }
+// Transpose of resetCellPeriodicFluxes and the wraps, as a gather: a point of the interior range of the
+// periodic axes collects the cotangents of its copies, the indices whose ghost_source it is (four on a
+// wrapped axis of four points, the smallest); they keep theirs, which the transposed
+// contravariantToCartesian does not read.  One thread per point next to the periodic boundaries, of three
+// components.  Bound by the launch: 13 us at 128 x 96 x 64 with two periodic axes, where the six launches
+// that scattered one axis and side at a time took 40.
+__device__ __forceinline__ int copies(int x, int m, int per, int (&c)[5]) {
+    int n = 0;
+    c[n++] = x;
+    if (per == TOSCA_PERIODIC_NONE) return n;
+    const int w = per == TOSCA_PERIODIC_WRAP ? GW : 0;
+    for (int y = -w; y <= 0; y++)
+        if (ghost_source(y, m, per, RESET_CELL) == x) c[n++] = y;
+    for (int y = m - 1; y < m + w; y++)
+        if (ghost_source(y, m, per, RESET_CELL) == x) c[n++] = y;
+    return n;
 }
-
-// transpose of k_reset_axis: boundary cells 0 / m-1 took cells m-2 / 1 over the owned range of the
-// other two axes
-__global__ void k_reset_axis_adj(double *a, int ncomp, Geo g, int axis) {
-    const int m[3] = {g.mx, g.my, g.mz};
-    const int t1 = (axis == 0) ? 1 : 0, t2 = (axis == 2) ? 1 : 2;
-    const int a1 = blockIdx.x * blockDim.x + threadIdx.x, a2 = blockIdx.y, side = blockIdx.z;
-    if (a1 >= m[t1] || a2 >= m[t2]) return;
-    int d[3], s[3];
-    d[axis] = side ? m[axis] - 1 : 0;
-    s[axis] = side ? 1 : m[axis] - 2;
-    d[t1] = s[t1] = a1;
-    d[t2] = s[t2] = a2;
-    copy_adj(a, ncomp, g.L(d[2], d[1], d[0]), g.L(s[2], s[1], s[0]));
-}
-
-// transpose of k_wrap_axis: ghost layers took the wrapped owned values, over the transverse ranges
-// that include the ghosts of the other type-2 axes.  One launch per side (layer0 = 0: the ghosts
-// below the axis, GW: above), so that the sources of one launch are distinct even on an axis of
-// fewer than 2 GW points.
-__global__ void k_wrap_axis_adj(double *a, int ncomp, Geo g, int axis, int layer0) {
-    const int m[3] = {g.mx, g.my, g.mz};
-    const int t1 = (axis == 0) ? 1 : 0, t2 = (axis == 2) ? 1 : 2;
-    const int lo1 = (g.per[t1] == TOSCA_PERIODIC_WRAP) ? -GW : 0, n1 = m[t1] + ((g.per[t1] == TOSCA_PERIODIC_WRAP) ? 2 * GW : 0);
-    const int lo2 = (g.per[t2] == TOSCA_PERIODIC_WRAP) ? -GW : 0, n2 = m[t2] + ((g.per[t2] == TOSCA_PERIODIC_WRAP) ? 2 * GW : 0);
-    const int a1 = blockIdx.x * blockDim.x + threadIdx.x, a2 = blockIdx.y, sl = layer0 + blockIdx.z;
-    if (a1 >= n1 || a2 >= n2) return;
-    const int n = m[axis];
-    const int dst = (sl < GW) ? (sl - GW) : (n + sl - GW);
-    const int src = (sl < GW) ? (n + sl - GW) : (sl - GW);
-    int d[3], s[3];
-    d[axis] = dst; s[axis] = src;
-    d[t1] = s[t1] = lo1 + a1;
-    d[t2] = s[t2] = lo2 + a2;
-    copy_adj(a, ncomp, g.L(d[2], d[1], d[0]), g.L(s[2], s[1], s[0]));
+__global__ void __launch_bounds__(256) k_ghosts_adj(double *a, Geo g, Shell S) {
+    int i, j, k, ci[5], cj[5], ck[5];
+    if (!shell_point(S, blockIdx.x * blockDim.x + threadIdx.x, i, j, k)) return;
+    const int ni = copies(i, g.mx, g.per[0], ci), nj = copies(j, g.my, g.per[1], cj), nk = copies(k, g.mz, g.per[2], ck);
+    if (ni * nj * nk == 1) return;
+    V3 s{0.0, 0.0, 0.0};
+    for (int r = 0; r < nk; r++)
+        for (int q = 0; q < nj; q++)
+            for (int p = 0; p < ni; p++) {
+                const V3 v = ld3(a, g.L(ck[r], cj[q], ci[p]));
+                s = V3{s.x + v.x, s.y + v.y, s.z + v.z};
+            }
+    st3(a, g.L(k, j, i), s);
 }
 
 // ucat = M^-1 q at an interior cell, M the rows csi, eta, zet: qbar = M^-T ucat_bar, by Cramer's
-// rule on M^T; written for the interior cells (every other point of qbar stays 0)
+// rule on M^T; written for the interior cells (nothing else of qbar is read)
 __global__ void k_c2c_adj_solve(const double *ubar, const double *csi, const double *eta, const double *zet,
                                 double *qbar, Geo g) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1, j = blockIdx.y * blockDim.y + threadIdx.y + 1,
@@ -124,69 +108,66 @@ __global__ void k_c2c_adj_solve(const double *ubar, const double *csi, const dou
 }
 
 // q_a of cell c averages the faces c - e_a and c of component a, so face p collects half of qbar_a
-// of the cells p and p + e_a (zero outside the interior cells); one thread per owned point
-__global__ void k_c2c_adj_gather(const double *qbar, double *vbar, Geo g) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y, k = blockIdx.z;
-    if (i > g.mx - 1) return;
+// of the cells p and p + e_a (zero outside the interior cells); added with vbar (the owned range of a local
+// cotangent) to the global xbar, one thread per owned point.  Bound by memory (96 bytes a point): 29 us at
+// 128 x 96 x 64, where clearing qbar, adding to vbar and adding vbar to xbar apart took 48
+__global__ void k_c2c_adj_gather(const double *qbar, const double *vbar, double *xbar, Geo g) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y * blockDim.y + threadIdx.y, k = blockIdx.z;
+    if (i > g.mx - 1 || j > g.my - 1) return;
     const long c = g.L(k, j, i);
-    vbar[3 * c + 0] = vbar[3 * c + 0] + 0.5 * (qbar[3 * c + 0] + qbar[3 * (long)g.L(k, j, i + 1) + 0]);
-    vbar[3 * c + 1] = vbar[3 * c + 1] + 0.5 * (qbar[3 * c + 1] + qbar[3 * (long)g.L(k, j + 1, i) + 1]);
-    vbar[3 * c + 2] = vbar[3 * c + 2] + 0.5 * (qbar[3 * c + 2] + qbar[3 * (long)g.L(k + 1, j, i) + 2]);
+    auto in = [](int x, int m) { return x >= 1 && x <= m - 2; };
+    const bool I = in(i, g.mx), J = in(j, g.my), K = in(k, g.mz);
+    auto q = [&](bool cell, int a, long p) { return cell ? qbar[3 * p + a] : 0.0; };
+    const V3 v = ld3(vbar, c);
+    double *x = xbar + 3 * gidx(g, k, j, i);
+    x[0] = x[0] + (v.x + 0.5 * (q(I && J && K, 0, c) + q(in(i + 1, g.mx) && J && K, 0, c + 1)));
+    x[1] = x[1] + (v.y + 0.5 * (q(I && J && K, 1, c) + q(I && in(j + 1, g.my) && K, 1, g.L(k, j + 1, i))));
+    x[2] = x[2] + (v.z + 0.5 * (q(I && J && K, 2, c) + q(I && J && in(k + 1, g.mz), 2, g.L(k + 1, j, i))));
 }
 
-// xbar (global) += the owned range of vbar (local); one thread per owned double
-__global__ void k_add_owned(double *xbar, const double *vbar, Geo g, long n) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    xbar[t] = xbar[t] + vbar[3 * owned_local(g, t / 3) + t % 3];
-}
-
-// transpose of the face-0 copy of a periodic axis on a global vector: plane 0 took plane m-2 over
-// the whole owned range of the other two axes (all three components)
-__global__ void k_face_periodic_adj(double *xbar, Geo g, int axis) {
+// Transpose of the ExplicitRhsU face resets on a global vector, with x the flux before them: plane 0 of
+// each periodic axis took plane m-2 over the whole owned range of the other two axes (all three
+// components), one axis after the other, so a point collects the cotangents of its copies, which keep none;
+// then the patches' rule (the same faces as the forward's).  Every point is written by one thread: the copies,
+// those with an index 0 on a periodic axis, by their source's
+__global__ void __launch_bounds__(256) k_face_resets_adj(double *xbar, const double *x, Geo g, PatchKinds P, Shell S) {
+    int q[3];
+    if (!shell_point(S, blockIdx.x * blockDim.x + threadIdx.x, q[0], q[1], q[2])) return;
     const int m[3] = {g.mx, g.my, g.mz};
-    const int t1 = (axis == 0) ? 1 : 0, t2 = (axis == 2) ? 1 : 2;
-    const int a1 = blockIdx.x * blockDim.x + threadIdx.x, a2 = blockIdx.y;
-    if (a1 >= m[t1] || a2 >= m[t2]) return;
-    int d[3], s[3];
-    d[axis] = 0;
-    s[axis] = m[axis] - 2;
-    d[t1] = s[t1] = a1;
-    d[t2] = s[t2] = a2;
-    const long cd = gidx(g, d[2], d[1], d[0]), cs = gidx(g, s[2], s[1], s[0]);
-    for (int q = 0; q < 3; q++) {
-        xbar[3 * cs + q] = xbar[3 * cs + q] + xbar[3 * cd + q];
-        xbar[3 * cd + q] = 0.0;
+    bool two[3], copy = false;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        const bool per = g.per[a] != TOSCA_PERIODIC_NONE;
+        copy = copy || (per && q[a] == 0);
+        two[a] = per && q[a] == m[a] - 2;
     }
-}
-
-// transpose of k_no_penetration on a global vector, with x the flux before the reset: one thread
-// per face of the six patches (the same faces and rules as the forward kernel)
-__global__ void k_no_penetration_adj(double *xbar, const double *x, Geo g, Kinds P) {
-    const int q = blockIdx.z, a = q >> 1, side = q & 1;
-    const int m[3] = {g.mx, g.my, g.mz};
-    const int t1 = (a == 0) ? 1 : 0, t2 = (a == 2) ? 1 : 2;
-    const int x1 = blockIdx.x * blockDim.x + threadIdx.x, x2 = blockIdx.y;
-    if (x1 >= m[t1] - 1 || x2 >= m[t2] - 1) return;
-    const int b = P.bc[q];
-    if (b != TOSCA_BCU_NOSLIP && b != TOSCA_BCU_WALLFUNCTION && b != TOSCA_BCU_SLIP && b != TOSCA_BCU_ZEROGRADIENT) return;
-    int idx[3];
-    idx[a] = side ? m[a] - 2 : 0;
-    idx[t1] = x1;
-    idx[t2] = x2;
-    const long o = 3 * gidx(g, idx[2], idx[1], idx[0]) + a;
-    if (b == TOSCA_BCU_ZEROGRADIENT) {
-        const double v = x[o];
-        if ((side == 0 && v > 0.0) || (side == 1 && v < 0.0)) xbar[o] = 0.0;
-    } else {
-        xbar[o] = 0.0;
+    if (copy) return;
+    double s[3] = {0.0, 0.0, 0.0};
+    for (int di = 0; di <= two[0]; di++)
+        for (int dj = 0; dj <= two[1]; dj++)
+            for (int dk = 0; dk <= two[2]; dk++) {
+                const long o = 3 * gidx(g, dk ? 0 : q[2], dj ? 0 : q[1], di ? 0 : q[0]);
+                for (int a = 0; a < 3; a++) {
+                    s[a] = s[a] + xbar[o + a];
+                    if (di | dj | dk) xbar[o + a] = 0.0;
+                }
+            }
+    const long o = 3 * gidx(g, q[2], q[1], q[0]);
+    const bool in = q[0] <= m[0] - 2 && q[1] <= m[1] - 2 && q[2] <= m[2] - 2;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+#pragma unroll
+        for (int side = 0; side < 2; side++) {
+            if (!in || q[a] != (side ? m[a] - 2 : 0)) continue;
+            const int b = P.bc[2 * a + side];
+            if (b == TOSCA_BCU_NOSLIP || b == TOSCA_BCU_WALLFUNCTION || b == TOSCA_BCU_SLIP) s[a] = 0.0;
+            else if (b == TOSCA_BCU_ZEROGRADIENT) {
+                const double v = x[o + a];
+                if (side == 0 ? v > 0.0 : v < 0.0) s[a] = 0.0;
+            }
+        }
+        xbar[o + a] = s[a];
     }
-}
-
-Kinds kinds_of(const tosca_params *p) {
-    Kinds K;
-    for (int q = 0; q < 6; q++) K.bc[q] = p->bc_u[q];
-    return K;
 }
 
 }  // namespace
@@ -205,53 +186,35 @@ void launch_rk3w_adj_combine(const double *xbar, double *carry, double *rbar, do
                  carry, rbar, a, b, n);
 }
 
-// transpose of launch_reset_cell_periodic (k_reset_axis on each periodic axis, then the wraps):
-// the wraps' transposes in reverse axis order, then the resets'
-void launch_reset_cell_periodic_adj(double *a, int ncomp, const Geo &g, hipStream_t s) {
+// transpose of launch_reset_cell_periodic on a vector field, for the interior cells
+void launch_reset_cell_periodic_adj(double *a, const Geo &g, hipStream_t s) {
+    // the points that have copies: up to GW from a wrapped end, the first and last interior cells otherwise;
+    // over the boundary cells of the other axes too, whose copies are no interior cells', nothing is needed
     const int m[3] = {g.mx, g.my, g.mz};
-    for (int axis = 2; axis >= 0; axis--) {
-        if (g.per[axis] != TOSCA_PERIODIC_WRAP) continue;
-        const int t1 = (axis == 0) ? 1 : 0, t2 = (axis == 2) ? 1 : 2;
-        const int n1 = m[t1] + ((g.per[t1] == TOSCA_PERIODIC_WRAP) ? 2 * GW : 0);
-        const int n2 = m[t2] + ((g.per[t2] == TOSCA_PERIODIC_WRAP) ? 2 * GW : 0);
-        for (int layer0 = GW; layer0 >= 0; layer0 -= GW)
-            TOSCA_LAUNCH("k_wrap_axis_adj", k_wrap_axis_adj, dim3((n1 + 127) / 128, n2, GW), dim3(128), 0, s, a, ncomp,
-                         g, axis, layer0);
+    int olo[3], ohi[3], clo[3], chi[3];
+    for (int q = 0; q < 3; q++) {
+        const bool per = g.per[q] != TOSCA_PERIODIC_NONE, wrap = g.per[q] == TOSCA_PERIODIC_WRAP;
+        olo[q] = 1; ohi[q] = m[q] - 1;
+        clo[q] = min(ohi[q], wrap ? GW : per ? 2 : 1);
+        chi[q] = max(clo[q], wrap ? m[q] - GW : per ? m[q] - 2 : m[q] - 1);
     }
-    for (int axis = 2; axis >= 0; axis--) {
-        if (g.per[axis] == TOSCA_PERIODIC_NONE) continue;
-        const int t1 = (axis == 0) ? 1 : 0, t2 = (axis == 2) ? 1 : 2;
-        TOSCA_LAUNCH("k_reset_axis_adj", k_reset_axis_adj, dim3((m[t1] + 127) / 128, m[t2], 2), dim3(128), 0, s, a, ncomp,
-                     g, axis);
-    }
+    const Shell S = make_shell(olo, ohi, clo, chi);
+    if (S.total) TOSCA_LAUNCH("k_ghosts_adj", k_ghosts_adj, dim3((S.total + 255) / 256), dim3(256), 0, s, a, g, S);
 }
 
-void launch_c2c_adj(const double *ubar, const tosca_mesh *m, double *qbar, double *vbar, const Geo &g, hipStream_t s) {
-    launch_fill(qbar, 3L * g.nloc(), 0.0, s);
+void launch_c2c_adj(const double *ubar, const tosca_mesh *m, double *qbar, const double *vbar, double *xbar, const Geo &g,
+                    hipStream_t s) {
     TOSCA_LAUNCH("k_c2c_adj_solve", k_c2c_adj_solve, dim3((g.mx - 2 + 63) / 64, (g.my - 2 + 3) / 4, g.mz - 2),
                  dim3(64, 4), 0, s, ubar, m->csi, m->eta, m->zet, qbar, g);
-    TOSCA_LAUNCH("k_c2c_adj_gather", k_c2c_adj_gather, dim3((g.mx + 255) / 256, g.my, g.mz), dim3(256), 0, s, qbar, vbar,
-                 g);
+    TOSCA_LAUNCH("k_c2c_adj_gather", k_c2c_adj_gather, dim3((g.mx + 63) / 64, (g.my + 3) / 4, g.mz), dim3(64, 4), 0, s, qbar, vbar,
+                 xbar, g);
 }
 
-void launch_add_owned(double *xbar, const double *vbar, const Geo &g, hipStream_t s) {
-    const long n = 3L * g.mx * g.my * g.mz;
-    TOSCA_LAUNCH("k_add_owned", k_add_owned, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, xbar, vbar, g, n);
-}
-
-// transpose of the ExplicitRhsU face resets y = Pf(Pn(x)) on a global cotangent: Pf's copies in
-// reverse axis order, then Pn's mask (x: the state before the resets)
+// transpose of the ExplicitRhsU face resets y = Pf(Pn(x)) on a global cotangent (x: the state before the resets)
 void launch_face_resets_adj(double *xbar, const double *x, const tosca_params *p, const Geo &g, hipStream_t s) {
-    const int m[3] = {g.mx, g.my, g.mz};
-    for (int axis = 2; axis >= 0; axis--) {
-        if (g.per[axis] == TOSCA_PERIODIC_NONE) continue;
-        const int t1 = (axis == 0) ? 1 : 0, t2 = (axis == 2) ? 1 : 2;
-        TOSCA_LAUNCH("k_face_periodic_adj", k_face_periodic_adj, dim3((m[t1] + 127) / 128, m[t2]), dim3(128), 0, s, xbar,
-                     g, axis);
-    }
-    const int n = std::max(g.mx, std::max(g.my, g.mz));
-    TOSCA_LAUNCH("k_no_penetration_adj", k_no_penetration_adj, dim3((n + 127) / 128, n, 6), dim3(128), 0, s, xbar, x, g,
-                 kinds_of(p));
+    const int zero[3] = {0, 0, 0}, own[3] = {g.mx, g.my, g.mz}, lo[3] = {1, 1, 1}, hi[3] = {g.mx - 2, g.my - 2, g.mz - 2};
+    const Shell S = make_shell(zero, own, lo, hi);
+    TOSCA_LAUNCH("k_face_resets_adj", k_face_resets_adj, dim3((S.total + 255) / 256), dim3(256), 0, s, xbar, x, g, patch_kinds(p), S);
 }
 
 }  // namespace tosca
