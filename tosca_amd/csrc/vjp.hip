@@ -128,7 +128,7 @@ struct VjpArgs {
     double *csbar;
     double *nutbar_acc; // nu_t given as an input: its cotangent is accumulated here (local)
     P *nueb[3];         // per face direction: cotangent of nu_eff at each face (n values)
-    P *rows;            // ucat cotangents summed per row: own, jp, jm, jpp (k_vjp_march), n vectors each
+    P *rows;            // ucat cotangents summed per row: own, and for rows of other workgroups jp, jm, jpp (n vectors each)
     double *tb;         // theta cotangents summed per row: the row's own, row j+1's (n values each)
     long n;
     double scale, bscale, tRef, nu;
@@ -358,8 +358,7 @@ __device__ __forceinline__ void boundary_face(const VjpArgs<T, P> &A, const Geo 
 // cotangents and the ucat cotangents of their regular stencils.
 //
 // A wave is one row j of 64 points along i and steps through the planes; lane 0 is point i0 - 2, and the
-// 60 lanes 2 .. 61 own their cell (a cell collects from the faces i-2 .. i+1).  Waves are independent
-// (no LDS, no barrier).  Each plane the thread evaluates the i, j and k face of its point: the
+// 60 lanes 2 .. 61 own their cell (a cell collects from the faces i-2 .. i+1).  Each plane the thread evaluates the i, j and k face of its point: the
 // convective cotangent cv = -V Fbar and the cotangents gc, ge, gz of the three derivative vectors.  A
 // face contributes to the cells
 //   normal derivative        left -gn, right +gn
@@ -367,35 +366,41 @@ __device__ __forceinline__ void boundary_face(const VjpArgs<T, P> &A, const Geo 
 //                            cell upwind of the pair)
 //   transverse derivatives   for both cells of the pair: +g/4 one up, -g/4 one down the transverse axis
 // and these are added where they land: along i by lane shifts, along k in the accumulators of four
-// planes, and only what goes to the neighbouring rows leaves the thread: per point the row's own sum
-// `own`, `jp` for row j+1, `jm` for row j-1 and (QUICK) `jpp` for row j+2, 9 or 12 values instead of
-// the 36 of three face packets.  k_vjp_finish adds the rows.  Buoyancy's theta cotangent comes along,
-// since its icsi.z, jeta.z, kzet.z are loaded here.
+// planes, and what goes to the neighbouring rows, `jp` for row j+1, `jm` for row j-1 and (QUICK) `jpp` for row
+// j+2, through LDS where that row is one of the workgroup's four (one barrier a plane) and to memory where it
+// is not: per point the row's own sum `own` and, at the workgroup's ends, jp of its last row, jm of its first,
+// jpp of its last two, on average 5 to 6 values instead of the 36 of three face packets.  k_vjp_finish adds the
+// rows.  Buoyancy's theta cotangent comes along, since its icsi.z, jeta.z, kzet.z are loaded here.
 //
-// Bound by memory: 504 bytes a point in FP64 (nine metric vectors 216, four arrays of row sums 96), about
-// 890 moved, since a wave's 64 points end within cache lines, 4 of them overlap and a chunk of planes loads 3
+// Bound by memory: 456 bytes a point in FP64 (nine metric vectors 216, row sums 48), about 840 moved, since a wave's 64 points end within cache lines, 4 of them overlap and a chunk of planes loads 3
 // more.  The registers (two waves a SIMD) hold the sums of four planes; the row sums and ucont_bar are
 // written as whole vectors, since stores of 8 of 24 bytes cost a pass over the line each.  Against a launch
 // that wrote the three packets of every face and a cell kernel that gathered them: the adjoint of the
-// 192 x 192 x 128 hill (FP64, QUICK) 2.60 -> 1.53 ms, of which this kernel is 0.82, and of the 384 x 256 x 96
-// box (mixed, central) 3.69 -> 2.07, of which 1.03.
+// 192 x 192 x 128 hill (FP64, QUICK) 2.60 -> 1.49 ms, of which this kernel is 0.84, and of the 384 x 256 x 96
+// box (mixed, central) 3.69 -> 1.94, of which 1.00.  Without the exchange in LDS every row's sums went to
+// memory: 1.52 and 2.06 (this kernel 0.82 and 1.03, k_vjp_finish 0.43 and 0.63 for 0.38 and 0.54); with
+// workgroups of eight rows 1.47 and 1.95, but 0.16 for 0.14 on the 128 x 96 x 64 grid, which they do not fill.
+constexpr int VM_NR = 4;         // rows of a workgroup
 template <class T, class P, bool QUICK>
-__global__ void __launch_bounds__(256, 2) k_vjp_march(VjpArgs<T, P> A, Geo g, int kchunk, int ti, int tj, int nbnd, int nmax) {
-    const int lane = threadIdx.x;
+__global__ void __launch_bounds__(64 * VM_NR, 2) k_vjp_march(VjpArgs<T, P> A, Geo g, int kchunk, int ti, int tj, int nbnd, int nmax) {
+    // per row of the workgroup: what it hands to the row above (jp, of plane t-1), to the row below (jm) and to
+    // the second row above (jpp), both of plane t and read a plane step later
+    __shared__ double sP[2][VM_NR][3][64], sM[3][VM_NR][3][64], sQ[QUICK ? 3 : 1][VM_NR][3][64];
+    const int lane = threadIdx.x, r = __builtin_amdgcn_readfirstlane(threadIdx.y);
     const int nm = gridDim.x - nbnd;
     if (blockIdx.x >= nm) {
-        boundary_face(A, g, ((blockIdx.x - nm) * 4 + threadIdx.y) * 64 + lane, nmax);
+        boundary_face(A, g, ((blockIdx.x - nm) * VM_NR + r) * 64 + lane, nmax);
         return;
     }
     const int tile = xcd_tile(blockIdx.x, nm);      // j fastest, then i, then the k chunk
     const int bj = tile % tj, bi = (tile / tj) % ti, bk = tile / (ti * tj);
-    const int j = 1 + bj * 4 + threadIdx.y, i = bi * 60 + lane - 2;
-    if (j > g.my - 2) return;                          // whole waves; the kernel has no barrier
+    const int jt = 1 + bj * VM_NR + r, i = bi * 60 + lane - 2, j = min(jt, g.my - 2);
+    const bool rowOk = jt <= g.my - 2;                 // rows past the end hand out zeros
     const int kb = bk * kchunk, ke = min(kb + kchunk, g.mz);     // cells [kb, ke)
     const int ia = min(max(i, 0), g.mx - 1);
     const int SJ = g.gxm, SK = g.gxm * g.gym, c0 = g.L(0, j, ia);
-    const bool mine = lane >= 2 && lane < 62 && i < g.mx;
-    const bool cellI = i >= 1 && i <= g.mx - 2;
+    const bool mine = lane >= 2 && lane < 62 && i < g.mx && rowOk;
+    const bool cellI = i >= 1 && i <= g.mx - 2 && rowOk;
     const bool okJ0 = cellI && j <= g.my - 3;
     const long n = A.n;
     P *own = A.rows, *jp = A.rows + 3 * n, *jm = A.rows + 6 * n, *jpp = A.rows + 9 * n;
@@ -407,6 +412,9 @@ __global__ void __launch_bounds__(256, 2) k_vjp_march(VjpArgs<T, P> A, Geo g, in
     // transverse-j cotangent of plane t-1, and the k face's theta cotangent of plane t-1
     V3 a0 = Z, a1 = Z, a2 = Z, a3 = Z, p0 = Z, p1 = Z, p2 = Z, tk = Z;
     double hk = 0.0;
+    auto put = [&](double (&d)[VM_NR][3][64], V3 v) { d[r][0][lane] = v.x; d[r][1][lane] = v.y; d[r][2][lane] = v.z; };
+    auto from = [&](const double (&d)[VM_NR][3][64], int q) { return V3{d[q][0][lane], d[q][1][lane], d[q][2][lane]}; };
+    int slot = 0, last = 2;                            // of planes t and t-1 in sM and sQ
     for (int t = kb - 2; t <= ke; t++) {
         const int tc = min(max(t, 0), g.mz - 1);
         const int c = opaque_index(c0 + tc * SK);
@@ -506,7 +514,9 @@ __global__ void __launch_bounds__(256, 2) k_vjp_march(VjpArgs<T, P> A, Geo g, in
             p1 = add3v(p1, add3v(add3v(sc3(wr, cv), G[1]), ld));
             if constexpr (QUICK) {
                 JM = sc3(pos ? -0.125 : 0.0, cv);
-                if (face) stp3(jpp, c, sc3(pos ? 0.0 : -0.125, cv));
+                const V3 q = sc3(pos ? 0.0 : -0.125, cv);
+                put(sQ[slot], q);
+                if (face && (r >= VM_NR - 2 || j >= g.my - 3)) stp3(jpp, c, q);
             }
             const V3 b = sc3(0.25, G[2]);
             a2 = add3v(a2, b);
@@ -553,14 +563,23 @@ __global__ void __launch_bounds__(256, 2) k_vjp_march(VjpArgs<T, P> A, Geo g, in
                 if (okJ) A.vbar[3 * c + 1] = T(vb.y);
                 if (okK) A.vbar[3 * c + 2] = T(vb.z);
             }
-            stp3(jm, c, JM);
+            if (r == 0) stp3(jm, c, JM);
             if (A.tbar) { A.tb[c] = h; A.tb[c + n] = hj; }
         }
+        put(sM[slot], JM);
+        put(sP[t & 1], p0);
+        __syncthreads();
+        V3 S = a0;
+        if (r >= 1) S = add3v(S, from(sP[t & 1], r - 1));
+        if (r < VM_NR - 1) S = add3v(S, from(sM[last], r + 1));
+        if constexpr (QUICK) { if (r >= 2) S = add3v(S, from(sQ[last], r - 2)); }
         if (t - 1 >= kb && t - 1 < ke && mine) {
             const int cm = opaque_index(c0 + (t - 1) * SK);
-            stp3(own, cm, a0);
-            stp3(jp, cm, p0);
+            stp3(own, cm, S);
+            if (r == VM_NR - 1 || j == g.my - 2) stp3(jp, cm, p0);
         }
+        last = slot;
+        slot = slot == 2 ? 0 : slot + 1;
         a0 = a1; a1 = a2; a2 = a3; a3 = Z;
         p0 = p1; p1 = p2; p2 = Z;
     }
@@ -568,7 +587,8 @@ __global__ void __launch_bounds__(256, 2) k_vjp_march(VjpArgs<T, P> A, Geo g, in
 
 namespace {
 // ucat_bar of point (i, j, k) from the boundary faces' scatter (which only reaches indices up to 2 from
-// either side) and the row sums of k_vjp_march: the row's own, row j-1's jp, row j+1's jm, row j-2's jpp
+// either side) and the row sums of k_vjp_march: the row's own and, from rows of another workgroup, row j-1's
+// jp, row j+1's jm, row j-2's jpp
 template <class T, class P>
 __device__ __forceinline__ V3 row_sums(const VjpArgs<T, P> &A, const Geo &g, int i, int j, int k, int c) {
     const long n = A.n;
@@ -576,10 +596,11 @@ __device__ __forceinline__ V3 row_sums(const VjpArgs<T, P> &A, const Geo &g, int
     auto get = [&](int q, int p) { return ldp3(A.rows + 3 * q * n, p); };
     V3 s{0, 0, 0};
     if (i <= 2 || i >= g.mx - 3 || j <= 2 || j >= g.my - 3 || k <= 2 || k >= g.mz - 3) s = cvt3<double>(ld3(A.ubar, c));
+    const int r = (j - 1) % VM_NR;                     // (of row 0: -1)
     if (j >= 1 && j <= jl) s = add3v(s, get(0, c));
-    if (j >= 2 && j <= jl + 1) s = add3v(s, get(1, c - SJ));
-    if (j <= jl - 1) s = add3v(s, get(2, c + SJ));
-    if (A.quick && j >= 3 && j <= jl + 2) s = add3v(s, get(3, c - 2 * SJ));
+    if (j >= 2 && j <= jl + 1 && (r == 0 || j == jl + 1)) s = add3v(s, get(1, c - SJ));
+    if (j <= jl - 1 && (r == VM_NR - 1 || j == 0)) s = add3v(s, get(2, c + SJ));
+    if (A.quick && j >= 3 && j <= jl + 1 && (r <= 1 || j == jl + 1)) s = add3v(s, get(3, c - 2 * SJ));
     return s;
 }
 // theta_bar of the point: the row's own part and row j-1's j face
@@ -616,10 +637,10 @@ __device__ __forceinline__ double w_own(bool np, int x, int m) { return np && x 
 // |S| path of the interior cells (nu_t_bar, Cs_bar, the cotangents of the three du_center vectors), which
 // a workgroup of 8 rows marching along k keeps on chip: along i by lane shifts, along j through LDS (one
 // barrier a plane), along k in the accumulators of three planes.  62 x 6 points a workgroup.
-// Bound by latency: 288 bytes a point in FP64, at 3.2 TB/s.  Every load of a cell is issued without a branch
-// (the six faces of nu_t_bar with a condition each took 0.49 ms on the 192 x 192 x 128 hill and 0.86 on the
-// mixed 384 x 256 x 96 box, 0.43 and 0.62 so); loading the row sums ahead of the barrier as well costs
-// 169 registers for 128 and with them half the waves: 0.50 ms.
+// Bound by latency: 240 bytes a point in FP64, at 3.0 TB/s; 0.38 ms on the 192 x 192 x 128 hill, 0.54 on the
+// mixed 384 x 256 x 96 box.  Every load of a cell is issued without a branch (with every row's sums read, the
+// six faces of nu_t_bar with a condition each took 0.49 and 0.86, 0.43 and 0.62 without); loading the row sums
+// ahead of the barrier as well cost 169 registers for 128 and with them half the waves: 0.50 ms.
 // ------------------------------------------------------------------------------------------------
 constexpr int VF_NR = 8, VF_TI = 62, VF_TJ = VF_NR - 2;
 template <class T, class P>
@@ -636,16 +657,9 @@ __global__ void __launch_bounds__(64 * VF_NR) k_vjp_finish(VjpArgs<T, P> A, Geo 
     const double wuI = w_up(np0, i, g.mx), wdI = w_dn(np0, i, g.mx), woI = w_own(np0, i, g.mx), woJ = w_own(np1, j, g.my);
     const double wuJ = w_up(np1, j - 1, g.my), wdJ = w_dn(np1, j + 1, g.my);     // of the rows below and above
     const int rm = max(r - 1, 0), rp = min(r + 1, VF_NR - 1);
-    const int SJ = g.gxm, SK = g.gxm * g.gym, jl = g.my - 2;
-    const long n = A.n;
+    const int SJ = g.gxm, SK = g.gxm * g.gym;
     const int p0 = g.L(0, min(j, g.my), min(i, g.mx));           // the point in plane 0 (indices from -1)
     const NuFaces fi = nu_faces(A, g, 0, i, 1), fj = nu_faces(A, g, 1, j, SJ);
-    const bool rOwn = j >= 1 && j <= jl, rJp = j >= 2 && j <= jl + 1, rJm = j <= jl - 1, rJpp = A.quick && j >= 3;
-    const bool edgeIJ = i <= 2 || i >= g.mx - 3 || j <= 2 || j >= g.my - 3;
-    auto get = [&](int q, bool ok, int p) {
-        const V3 v = ldp3(A.rows + 3 * q * n, p);
-        return V3{ok ? v.x : 0.0, ok ? v.y : 0.0, ok ? v.z : 0.0};
-    };
     V3 c0{0, 0, 0}, c1{0, 0, 0}, c2{0, 0, 0};          // sums of the points of planes k-1, k, k+1
     Vec3<T> um = ld3(A.ucat, p0 + (kb - 2) * SK), u = ld3(A.ucat, p0 + (kb - 1) * SK);
     for (int k = kb - 1; k <= ke; k++) {
@@ -776,13 +790,13 @@ void vjp_rhs_impl(const Geo &g, const tosca_mesh *mesh, const tosca_params *p, c
     } else {
         TOSCA_LAUNCH(f32 ? "k_vjp_fp_f32" : "k_vjp_fp", (k_vjp_fp<T, P>), cg, cb, 0, s, A, g);
     }
-    const int ti = (g.mx + 59) / 60, tj = (g.my - 2 + 3) / 4;
+    const int ti = (g.mx + 59) / 60, tj = (g.my - 2 + VM_NR - 1) / VM_NR;
     const int kc = plane_chunk(g.mz, ti * tj, 2 * NUM_CU, 3, 2000.0);
     const int nmax = max(g.my * g.mz, max(g.mx * g.mz, g.mx * g.my));
-    const int nbnd = (6 * nmax + 2047) / 2048 * 8;     // workgroups of 256 boundary faces, a multiple of the XCDs
+    const int nbnd = (6 * nmax + 64 * VM_NR * NUM_XCD - 1) / (64 * VM_NR * NUM_XCD) * NUM_XCD;     // a multiple of the XCDs
     const dim3 mg(nbnd + ti * tj * ((g.mz + kc - 1) / kc));
-    if (A.quick) TOSCA_LAUNCH(f32 ? "k_vjp_march_f32" : "k_vjp_march", (k_vjp_march<T, P, true>), mg, dim3(64, 4), 0, s, A, g, kc, ti, tj, nbnd, nmax);
-    else TOSCA_LAUNCH(f32 ? "k_vjp_march_f32" : "k_vjp_march", (k_vjp_march<T, P, false>), mg, dim3(64, 4), 0, s, A, g, kc, ti, tj, nbnd, nmax);
+    if (A.quick) TOSCA_LAUNCH(f32 ? "k_vjp_march_f32" : "k_vjp_march", (k_vjp_march<T, P, true>), mg, dim3(64, VM_NR), 0, s, A, g, kc, ti, tj, nbnd, nmax);
+    else TOSCA_LAUNCH(f32 ? "k_vjp_march_f32" : "k_vjp_march", (k_vjp_march<T, P, false>), mg, dim3(64, VM_NR), 0, s, A, g, kc, ti, tj, nbnd, nmax);
     if (renut) {
         const int fi = (g.mx + VF_TI - 1) / VF_TI, fj = (g.my + VF_TJ - 1) / VF_TJ;
         const int fc = plane_chunk(g.mz, fi * fj, 2 * NUM_CU, 2, 500.0);
