@@ -363,7 +363,8 @@ __device__ __forceinline__ void boundary_face(const VjpArgs<T, P> &A, const Geo 
 // face contributes to the cells
 //   normal derivative        left -gn, right +gn
 //   convective interpolation left and right (QUICK: left 3/4 or 3/8, right 3/8 or 3/4, and -1/8 of the
-//                            cell upwind of the pair)
+//                            cell upwind of the pair; the other end takes nothing, by selection, so that a value
+//                            that is not finite reaches the cells of the stencil alone)
 //   transverse derivatives   for both cells of the pair: +g/4 one up, -g/4 one down the transverse axis
 // and these are added where they land: along i by lane shifts, along k in the accumulators of four
 // planes, and what goes to the neighbouring rows, `jp` for row j+1, `jm` for row j-1 and (QUICK) `jpp` for row
@@ -482,8 +483,8 @@ __global__ void __launch_bounds__(64 * VM_NR, 2) k_vjp_march(VjpArgs<T, P> A, Ge
             const double wl = QUICK ? (pos ? 0.75 : 0.375) : 0.5, wr = QUICK ? (pos ? 0.375 : 0.75) : 0.5;
             V3 r = add3v(sc3(wr, cv), G[0]);
             if constexpr (QUICK) {
-                r = add3v(r, up(sc3(pos ? 0.0 : -0.125, cv)));
-                a1 = add3v(a1, dn(sc3(pos ? -0.125 : 0.0, cv)));
+                r = add3v(r, up(sel(!pos, sc3(-0.125, cv))));
+                a1 = add3v(a1, dn(sel(pos, sc3(-0.125, cv))));
             }
             a1 = add3v(a1, add3v(add3v(sc3(wl, cv), sc3(-1.0, G[0])), up(r)));
             T0 = add3v(T0, sc3(0.25, add3v(G[1], up(G[1]))));
@@ -513,8 +514,10 @@ __global__ void __launch_bounds__(64 * VM_NR, 2) k_vjp_march(VjpArgs<T, P> A, Ge
             a1 = add3v(a1, add3v(add3v(sc3(wl, cv), sc3(-1.0, G[1])), ld));
             p1 = add3v(p1, add3v(add3v(sc3(wr, cv), G[1]), ld));
             if constexpr (QUICK) {
-                JM = sc3(pos ? -0.125 : 0.0, cv);
-                const V3 q = sc3(pos ? 0.0 : -0.125, cv);
+                // (selected before the weights: behind them it took the FP64 instance from 10 spilled registers to 18)
+                const V3 cl = sel(pos, cv), cr = sel(!pos, cv);
+                JM = sc3(pos ? -0.125 : 0.0, cl);
+                const V3 q = sc3(-0.125, cr);
                 put(sQ[slot], q);
                 if (face && (r >= VM_NR - 2 || j >= g.my - 3)) stp3(jpp, c, q);
             }
@@ -545,8 +548,8 @@ __global__ void __launch_bounds__(64 * VM_NR, 2) k_vjp_march(VjpArgs<T, P> A, Ge
             a1 = add3v(a1, add3v(add3v(sc3(wl, cv), sc3(-1.0, G[2])), ld));
             a2 = add3v(a2, add3v(add3v(sc3(wr, cv), G[2]), ld));
             if constexpr (QUICK) {
-                a0 = add3v(a0, sc3(pos ? -0.125 : 0.0, cv));
-                a3 = sc3(pos ? 0.0 : -0.125, cv);
+                a0 = add3v(a0, sel(pos, sc3(-0.125, cv)));
+                a3 = sel(!pos, sc3(-0.125, cv));
             }
             tk = sc3(0.25, G[1]);
             T0 = add3v(T0, tk);
@@ -630,6 +633,8 @@ __device__ __forceinline__ NuFaces nu_faces(const A_ &A, const Geo &g, int q, in
 __device__ __forceinline__ double w_up(bool np, int x, int m) { return np && x == m - 2 ? 0.0 : np && x == 1 ? 1.0 : 0.5; }
 __device__ __forceinline__ double w_dn(bool np, int x, int m) { return np && x == m - 2 ? -1.0 : np && x == 1 ? 0.0 : -0.5; }
 __device__ __forceinline__ double w_own(bool np, int x, int m) { return np && x == m - 2 ? 1.0 : np && x == 1 ? -1.0 : 0.0; }
+// such a weight times v; a weight of zero takes nothing, also of a v that is not finite
+__device__ __forceinline__ V3 wt3(double w, V3 v) { return V3{w != 0.0 ? w * v.x : 0.0, w != 0.0 ? w * v.y : 0.0, w != 0.0 ? w * v.z : 0.0}; }
 }  // namespace
 
 // ------------------------------------------------------------------------------------------------
@@ -640,11 +645,12 @@ __device__ __forceinline__ double w_own(bool np, int x, int m) { return np && x 
 // Bound by latency: 240 bytes a point in FP64, at 3.0 TB/s; 0.38 ms on the 192 x 192 x 128 hill, 0.54 on the
 // mixed 384 x 256 x 96 box.  Every load of a cell is issued without a branch (with every row's sums read, the
 // six faces of nu_t_bar with a condition each took 0.49 and 0.86, 0.43 and 0.62 without); loading the row sums
-// ahead of the barrier as well cost 169 registers for 128 and with them half the waves: 0.50 ms.
+// ahead of the barrier as well cost 169 registers for 128 and with them half the waves: 0.50 ms.  The launch
+// bound holds it at 128 (132 of the compiler's own choice would leave three waves a SIMD).
 // ------------------------------------------------------------------------------------------------
 constexpr int VF_NR = 8, VF_TI = 62, VF_TJ = VF_NR - 2;
 template <class T, class P>
-__global__ void __launch_bounds__(64 * VF_NR) k_vjp_finish(VjpArgs<T, P> A, Geo g, int kchunk) {
+__global__ void __launch_bounds__(64 * VF_NR, 4) k_vjp_finish(VjpArgs<T, P> A, Geo g, int kchunk) {
     __shared__ double sG[2][3][VF_NR][64];
     const int lane = threadIdx.x, r = threadIdx.y;
     const int tile = xcd_tile();                       // j fastest, then i, then the k chunk
@@ -698,14 +704,13 @@ __global__ void __launch_bounds__(64 * VF_NR) k_vjp_finish(VjpArgs<T, P> A, Geo 
         sG[buf][0][r][lane] = ge.x; sG[buf][1][r][lane] = ge.y; sG[buf][2][r][lane] = ge.z;
         // own cell, then the cells along i
         const double woK = w_own(np2, k, g.mz);
-        c1 = add3v(c1, add3v(sc3(woI, gc), add3v(sc3(woJ, ge), sc3(woK, gz))));
-        c1 = add3v(c1, add3v(shup3(sc3(wuI, gc)), shdn3(sc3(wdI, gc))));
-        c2 = add3v(c2, sc3(w_up(np2, k, g.mz), gz));
-        c0 = add3v(c0, sc3(w_dn(np2, k, g.mz), gz));
+        c1 = add3v(c1, add3v(wt3(woI, gc), add3v(wt3(woJ, ge), wt3(woK, gz))));
+        c1 = add3v(c1, add3v(shup3(wt3(wuI, gc)), shdn3(wt3(wdI, gc))));
+        c2 = add3v(c2, wt3(w_up(np2, k, g.mz), gz));
+        c0 = add3v(c0, wt3(w_dn(np2, k, g.mz), gz));
         __syncthreads();                               // the other buffer is rewritten behind the next one
-        c1 = add3v(c1, V3{wuJ * sG[buf][0][rm][lane] + wdJ * sG[buf][0][rp][lane],
-                          wuJ * sG[buf][1][rm][lane] + wdJ * sG[buf][1][rp][lane],
-                          wuJ * sG[buf][2][rm][lane] + wdJ * sG[buf][2][rp][lane]});
+        c1 = add3v(c1, add3v(wt3(wuJ, V3{sG[buf][0][rm][lane], sG[buf][1][rm][lane], sG[buf][2][rm][lane]}),
+                             wt3(wdJ, V3{sG[buf][0][rp][lane], sG[buf][1][rp][lane], sG[buf][2][rp][lane]})));
         if (mine && k - 1 >= kb && k - 1 < ke) {       // the points of plane k-1 are complete
             const int cm = opaque_index(p0 + (k - 1) * SK);
             stp3(A.ubar, cm, add3v(row_sums(A, g, i, j, k - 1, cm), c0));
