@@ -63,7 +63,7 @@ __global__ void __launch_bounds__(256) k_face_resets(double *ucont, Geo g, Patch
 #pragma unroll
     for (int a = 0; a < 3; a++) {
         const double v = u[a], w = no_penetration(g, P, i, j, k, a, v);
-        if (w != v) u[a] = w;
+        if (__double_as_longlong(w) != __double_as_longlong(v)) u[a] = w;      // (as bits: -0.0 becomes 0.0)
     }
 }
 
