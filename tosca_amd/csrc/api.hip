@@ -227,6 +227,12 @@ int ensure_ws(tosca_ctx *c, size_t elems) {
     return TOSCA_OK;
 }
 
+// whether two arrays share memory (b may be null)
+bool overlap(const void *a, size_t na, const void *b, size_t nb) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return b && x < y + nb && y < x + na;
+}
+
 int launched(tosca_ctx *c, const char *what) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_err(c, TOSCA_ERR_DEVICE, "%s: %s", what, hipGetErrorString(e));
@@ -1271,7 +1277,26 @@ int tosca_formt(tosca_ctx *c, const tosca_mesh *m, const tosca_params *p, const 
             (rc = check_dev(c, tp->q_wall_j, 3 * (size_t)g.mz * g.mx * sizeof(double), "q_wall_j")))
             return rc;
     }
-    tosca::formt(g, m, p, tp, ucont, theta, nut, kt, rhs, scale, form_mode, c->stream);
+    // One launch reads the inputs and writes rhs, so an rhs in the memory of an input is formed in the
+    // workspace: its own values first (the boundary cells keep them), the result back behind the launch
+    double *out = rhs;
+    const size_t v = 3 * n * sizeof(double), sc = n * sizeof(double);
+    const struct { const double *p; size_t bytes; } in[] = {
+        {ucont, v}, {theta, sc}, {les ? nut : nullptr, sc}, {les ? kt : nullptr, sc}, {m->icsi, v}, {m->ieta, v}, {m->izet, v},
+        {m->jcsi, v}, {m->jeta, v}, {m->jzet, v}, {m->kcsi, v}, {m->keta, v}, {m->kzet, v}, {m->iaj, sc}, {m->jaj, sc},
+        {m->kaj, sc}, {m->aj, sc}, {les ? tp->q_wall_i : nullptr, 3 * (size_t)g.mz * g.my * sizeof(double)},
+        {les ? tp->q_wall_j : nullptr, 3 * (size_t)g.mz * g.mx * sizeof(double)}};
+    for (const auto &a : in)
+        if (overlap(rhs, ng, a.p, a.bytes)) out = nullptr;
+    if (!out) {
+        if ((rc = ensure_ws(c, ng / sizeof(double)))) return rc;
+        out = c->ws;
+        if (hipMemcpyAsync(out, rhs, ng, hipMemcpyDeviceToDevice, c->stream) != hipSuccess)
+            return set_err(c, TOSCA_ERR_DEVICE, "FormT: copy failed");
+    }
+    tosca::formt(g, m, p, tp, ucont, theta, nut, kt, out, scale, form_mode, c->stream);
+    if (out != rhs && hipMemcpyAsync(rhs, out, ng, hipMemcpyDeviceToDevice, c->stream) != hipSuccess)
+        return set_err(c, TOSCA_ERR_DEVICE, "FormT: copy failed");
     return launched(c, "FormT");
 }
 
