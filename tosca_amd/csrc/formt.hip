@@ -297,7 +297,7 @@ void formt(const Geo &g, const tosca_mesh *m, const tosca_params *p, const tosca
     FormTArgs A = formt_args(g, m, p, tp, ucont, theta, nut, kt);
     A.rhs = rhs; A.scale = scale; A.mode = mode;
     const int ti = (g.mx - 2 + FT_TI - 1) / FT_TI, tj = (g.my - 2 + FT_TJ - 1) / FT_TJ;
-    const int kc = plane_chunk(g.mz - 2, ti * tj, 2 * NUM_CU, 1, 500.0);
+    const int kc = plane_chunk(g.mz - 2, ti * tj, CHUNK_FORMT);
     const dim3 grid(ti, tj, (g.mz - 2 + kc - 1) / kc), block(64, FT_NR);
     if (!p->les_active) TOSCA_LAUNCH("k_formt", k_formt<KAP_NONE>, grid, block, 0, s, A, g, kc);
     else if (kt_model(p->les_model)) TOSCA_LAUNCH("k_formt", k_formt<KAP_KT>, grid, block, 0, s, A, g, kc);

@@ -4,29 +4,10 @@
 // reference-structured kernel.
 #pragma once
 
+#include "chunks.h"
 #include "kernels.h"
 
 namespace tosca {
-
-// k planes per chunk of a k-marching launch over `tiles` column tiles.  Workgroups run `slots` at a
-// time, each for its planes plus `over` plane steps of priming, so the launch takes about
-// ceil(tiles chunks / slots) (planes + over) plane steps, and neighbouring tiles drift apart along k,
-// so that they share fewer of their halo lines in L2: 1 + planes / drift per step.  The chunk count
-// that makes the product least, the smallest one where several do.  Large grids get whole rounds of
-// the chip (the 512 x 512 x 192 shard: FormU 8 chunks of 64 planes, 7.9 rounds, 4.99 ms; 5.31 in one
-// chunk, 5.42 in 24); grids with few columns get chunks short enough to occupy it (64^3 FormU 58 us,
-// 69 with the 8-plane chunks it had; 256 x 128 x 96 hill 0.39 ms, 0.47; 16 x 10 x 8 hill 21 us, 65).
-constexpr int NUM_CU = 256;
-inline int plane_chunk(int nk, int tiles, int slots, int over, double drift) {
-    double best = -1.0;
-    int kc = nk;
-    for (int c = 1; c <= nk; c++) {
-        const int k = (nk + c - 1) / c, n = (nk + k - 1) / k;
-        const double cost = (double)(((long)tiles * n + slots - 1) / slots) * (k + over) * (1.0 + k / drift);
-        if (best < 0.0 || cost < best) { best = cost; kc = k; }
-    }
-    return kc;
-}
 
 // T is the type of the flow fields (ucont, ucat, nut, theta): double on the FP64 path, float on
 // the mixed path.  Metrics, Jacobians, the wall stresses and the outputs are always double.

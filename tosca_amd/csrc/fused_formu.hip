@@ -713,7 +713,7 @@ void fused_formu(const Geo &g, const FormUArgsT<T, MT> &A, double *ws, hipStream
 
     const int nk = g.mz - 2;
     const int tiles = ((g.mx - 2 + TI - 1) / TI) * ((g.my - 2 + TJ - 1) / TJ);
-    const int kchunk = plane_chunk(nk, tiles, NUM_CU, 3, 2000.0), chunks = (nk + kchunk - 1) / kchunk;
+    const int kchunk = plane_chunk(nk, tiles, CHUNK_FORMU), chunks = (nk + kchunk - 1) / kchunk;
     dim3 grid((g.mx - 2 + TI - 1) / TI, (g.my - 2 + TJ - 1) / TJ, chunks);
     const char *kname = sizeof(T) == 8 ? "k_fused_formu" : sizeof(MT) == 8 ? "k_fused_formu_f32" : "k_fused_formu_f32m";
     // the cell bases formed from the face bases on FP64 metrics only (on the FP32 copies, whose

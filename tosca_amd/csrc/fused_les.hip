@@ -867,7 +867,7 @@ FilterShape filter_shape(const Geo &g) {
     const int nk = g.mz - 2;
     d.ti = (g.mx - 2 + FT::TI - 1) / FT::TI;
     d.tj = (g.my - 2 + FT::TJ - 1) / FT::TJ;
-    d.kchunk = plane_chunk(nk, d.ti * d.tj, NUM_CU, 2 * H + 1, 2e4);
+    d.kchunk = plane_chunk(nk, d.ti * d.tj, H == 1 ? CHUNK_FILTER3 : CHUNK_FILTER5);
     d.chunks = (nk + d.kchunk - 1) / d.kchunk;
     return d;
 }
@@ -891,7 +891,7 @@ void launch_dsm_lm_f32(const Geo &g, const tosca_mesh *m, const float *ucat, dou
     // as plane_chunk finds, so that the pieces do not change the rounding of the shifted sums
     const int chunks = max(1, min((2048 + ti * tj - 1) / (ti * tj), nk / 8));
     const int kref = (nk + chunks - 1) / chunks, nref = (nk + kref - 1) / kref;
-    const int kchunk = plane_chunk(kref, ti * tj * nref, NUM_CU, 2, 2e4);
+    const int kchunk = plane_chunk(kref, ti * tj * nref, CHUNK_FILTER_F32);
     const dim3 grid(ti, tj, nref * ((kref + kchunk - 1) / kchunk)), blk(64, DSM_NR);
     if (m32)
         TOSCA_LAUNCH("k_dsm_lm_f32m", k_dsm_lm_f32<float>, grid, blk, 0, s, g, ucat, m32->csi, m32->eta, m32->zet, m->aj, LM,
@@ -908,7 +908,7 @@ DpasdK dpasd_k_shape(const Geo &g) {
     const int nk = g.mz - 2;
     d.ti = (g.mx - 2 + DK_X - 1) / DK_X;
     d.tj = (g.my - 2 + DK_Y - 1) / DK_Y;
-    d.kchunk = plane_chunk(nk, d.ti * d.tj, 4 * NUM_CU, 2, 500.0);
+    d.kchunk = plane_chunk(nk, d.ti * d.tj, CHUNK_DPASD_K);
     d.chunks = (nk + d.kchunk - 1) / d.kchunk;
     return d;
 }
@@ -950,7 +950,7 @@ void fused_dpasd(const Geo &g, const tosca_mesh *m, const T *ucat, double maxCs,
         float *X = reinterpret_cast<float *>(ws + w.X);
         launch_dsm_lm_f32(g, m, ucat, LM, MM, Sabs, s, nullptr);
         const int nk = g.mz - 2, ti = (g.mx - 2 + DP_TI - 1) / DP_TI, tj = (g.my - 2 + DP_TJ - 1) / DP_TJ;
-        const int kchunk = plane_chunk(nk, ti * tj, NUM_CU, 1, 2000.0);
+        const int kchunk = plane_chunk(nk, ti * tj, CHUNK_DPASD_IJ);
         TOSCA_LAUNCH("k_dpasd_ij_f32", k_dpasd_ij_f32, dim3(ti, tj, (nk + kchunk - 1) / kchunk), dim3(64, DP_NR), 0, s, g,
                      ucat, m->csi, m->eta, m->zet, m->aj, X, nI, kchunk);
         const DpasdK d = dpasd_k_shape(g);
@@ -974,7 +974,7 @@ void fused_dsm(const Geo &g, const tosca_mesh *m, const T *ucat, double maxCs, d
     if constexpr (std::is_same<T, float>::value) launch_dsm_lm_f32(g, m, ucat, LM, MM, Sabs, s, m32);
     else launch_filter<1, false>(g, m, ucat, LM, MM, Sabs, nullptr, s);
     const int ctiles = ((g.mx - 2 + CX - 1) / CX) * ((g.my - 2 + CY - 1) / CY);
-    const int ckchunk = plane_chunk(nk, ctiles, 2 * NUM_CU, 2, 500.0), cchunks = (nk + ckchunk - 1) / ckchunk;
+    const int ckchunk = plane_chunk(nk, ctiles, CHUNK_BOX), cchunks = (nk + ckchunk - 1) / ckchunk;
     TOSCA_LAUNCH(sizeof(T) == 8 ? "k_dsm_cs_nut" : "k_dsm_cs_nut_f32", k_dsm_cs_nut<T>,
                  dim3((g.mx - 2 + CX - 1) / CX, (g.my - 2 + CY - 1) / CY, cchunks), dim3(CX, CY), 0, s, g, LM, MM, Sabs,
                  m->aj, maxCs, cs, nut, ckchunk);

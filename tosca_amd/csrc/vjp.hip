@@ -796,7 +796,7 @@ void vjp_rhs_impl(const Geo &g, const tosca_mesh *mesh, const tosca_params *p, c
         TOSCA_LAUNCH(f32 ? "k_vjp_fp_f32" : "k_vjp_fp", (k_vjp_fp<T, P>), cg, cb, 0, s, A, g);
     }
     const int ti = (g.mx + 59) / 60, tj = (g.my - 2 + VM_NR - 1) / VM_NR;
-    const int kc = plane_chunk(g.mz, ti * tj, 2 * NUM_CU, 3, 2000.0);
+    const int kc = plane_chunk(g.mz, ti * tj, CHUNK_VJP_MARCH);
     const int nmax = max(g.my * g.mz, max(g.mx * g.mz, g.mx * g.my));
     const int nbnd = (6 * nmax + 64 * VM_NR * NUM_XCD - 1) / (64 * VM_NR * NUM_XCD) * NUM_XCD;     // a multiple of the XCDs
     const dim3 mg(nbnd + ti * tj * ((g.mz + kc - 1) / kc));
@@ -804,7 +804,7 @@ void vjp_rhs_impl(const Geo &g, const tosca_mesh *mesh, const tosca_params *p, c
     else TOSCA_LAUNCH(f32 ? "k_vjp_march_f32" : "k_vjp_march", (k_vjp_march<T, P, false>), mg, dim3(64, VM_NR), 0, s, A, g, kc, ti, tj, nbnd, nmax);
     if (renut) {
         const int fi = (g.mx + VF_TI - 1) / VF_TI, fj = (g.my + VF_TJ - 1) / VF_TJ;
-        const int fc = plane_chunk(g.mz, fi * fj, 2 * NUM_CU, 2, 500.0);
+        const int fc = plane_chunk(g.mz, fi * fj, CHUNK_VJP_FINISH);
         TOSCA_LAUNCH(f32 ? "k_vjp_finish_f32" : "k_vjp_finish", (k_vjp_finish<T, P>), dim3(fi, fj, (g.mz + fc - 1) / fc),
                      dim3(64, VF_NR), 0, s, A, g, fc);
     } else {
