@@ -284,8 +284,8 @@ int tosca_rhs_vjp(tosca_ctx *ctx, const tosca_mesh *mesh, const tosca_params *pa
  * in; cs (local), rbar (global) FP64; ucont_bar, ucat_bar, theta_bar (local, FP32) and cs_bar
  * (local, FP64) overwritten.  The forward intermediates (nu_t, |S|, the face gradients and
  * interpolated velocities) are recomputed in FP32 as the mixed step computes them; the cotangent
- * arithmetic is FP64; the cotangent packets between the kernels are stored in FP32, which halves
- * their HBM traffic.  Same function, error codes and conventions as tosca_rhs_vjp. */
+ * arithmetic is FP64; the ucat cotangents that pass between the kernels are stored in FP32, which
+ * halves their HBM traffic.  Same function, error codes and conventions as tosca_rhs_vjp. */
 int tosca_rhs_vjp_mixed(tosca_ctx *ctx, const tosca_mesh *mesh, const tosca_params *params,
                         const float *ucont, const float *ucat, const float *theta, const double *cs,
                         const double *rbar, double scale, double buoy_scale,

@@ -88,7 +88,7 @@ __device__ __forceinline__ V3 contra_to_cart(const double *ucont, const double *
 
 // ucat at the interior cells, then resetCellPeriodicFluxes and the ghost wraps: the points B of the
 // periodic copies evaluate their source cell themselves, or copy it where it is no interior cell.  Bound by
-// memory: 120 bytes a cell at 4.6 TB/s, 0.137 ms for 0.136 + 0.013 in two launches at 256 x 192 x 96.  The
+// memory: 120 bytes a cell (155 moved) at 4.2 TB/s, 0.136 ms for 0.136 + 0.013 in two launches at 256 x 192 x 96.  The
 // last nint workgroups take 64 x 4 cells of a plane, the others, first for their scattered loads, 256 points of B
 __global__ void __launch_bounds__(256) k_contra_to_cart(const double *ucont, const double *csi, const double *eta, const double *zet,
                                  double *ucat, Geo g, int nbi, int nbj, int nint, Shell B) {

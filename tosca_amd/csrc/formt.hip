@@ -166,10 +166,10 @@ __device__ __forceinline__ double across_of(bool edge, int x, int m, double hp, 
 // rows j-1 and j+1 at k+1, row j+2 at k), the others from the planes before and the lanes beside, so that
 // lanes 2 .. 61 own cells.  Face 0 of a periodic axis is evaluated as face m-2, which
 // resetFacePeriodicFluxesVector copies there.
-// Bound by the loads: 288 bytes a point at 4.0 TB/s, 128 registers (four waves a SIMD).  384 x 256 x 128,
+// Bound by the loads: 296 bytes a point at 4.0 TB/s, 128 registers (four waves a SIMD).  384 x 256 x 128,
 // k_t: 1.27 ms as a face kernel that stored both fluxes of every face (0.95), twelve ghost launches on them
 // and a budget kernel; 1.06 in one launch with theta loaded for each face (36 loads, whose L1 lines were a
-// third of the kernel's); 0.95 so.  nu_t over the turbulent Prandtl number: 1.36, 1.28, 1.05 (with pow() for
+// third of the kernel's); 0.93 so.  nu_t over the turbulent Prandtl number: 1.36, 1.28, 1.05 (with pow() for
 // the cube root of the volume its constants, kept in registers across the planes, took 174 registers: 1.35).
 // The closure is a template parameter for the same reason.  Rows of 4 measured 0.98.
 // rhs = scale ((formMode != 2 ? div budget : 0) + (formMode != 1 ? visc budget : 0)) aj, interior

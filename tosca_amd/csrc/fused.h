@@ -71,9 +71,9 @@ void vjp_rhs(const Geo &g, const tosca_mesh *mesh, const tosca_params *p, const 
              const double *theta, const double *cs, const double *rbar, double scale, double buoy_scale,
              double *ucont_bar, double *ucat_bar, double *theta_bar, double *cs_bar, double *ws, hipStream_t s);
 
-// The same adjoint with FP32 flow fields and FP32 cotangent packets (the mixed step's function):
+// The same adjoint with FP32 flow fields (the mixed step's function):
 // the forward intermediates in FP32 as the mixed step computes them, the cotangent arithmetic in
-// FP64, the packets and intermediates stored in FP32, ucont_bar / ucat_bar / theta_bar FP32.
+// FP64, what passes between the kernels (theta's sums apart) and ucont_bar / ucat_bar / theta_bar in FP32.
 void vjp_rhs_mixed(const Geo &g, const tosca_mesh *mesh, const tosca_params *p, const float *ucont, const float *ucat,
                    const double *cs, const double *rbar, double scale, double buoy_scale, float *ucont_bar,
                    float *ucat_bar, float *theta_bar, double *cs_bar, double *ws, hipStream_t s);

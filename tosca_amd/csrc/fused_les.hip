@@ -141,7 +141,9 @@ __device__ __forceinline__ void tile_shift(const T *ucat, const MT *csi, const M
 // point; the 28 quantities are filtered along i across the lanes of the wave, along j through LDS and
 // along k as two planes of partial sums in registers.  MT: storage type of csi, eta, zet (float: the
 // FP32 metric copies of the mixed step that runs FormU on them; the strain uses FP32 metrics either
-// way)
+// way).  The axes in this order and not k first, as FP64 takes them: another order of the FP32 sums
+// moves Cs by their rounding (5e-7), in outputs that callers hold as FP64.  On the 512 x 512 x 192 shard
+// 2.38 ms where the FP64 kernel takes 2.67; DPASD's three FP32 kernels 2.38 + 3.5 + 2.8, FP64's two 2.67 + 4.84
 template <class MT>
 __global__ void __launch_bounds__(64 * DSM_NR) k_dsm_lm_f32(Geo g, const float *ucat, const MT *csi,
                                                             const MT *eta, const MT *zet, const double *aj,

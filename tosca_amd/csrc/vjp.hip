@@ -95,34 +95,16 @@ __device__ void du_k_adj(const Geo &g, T *ub, int i, int j, int k, V3 gc, V3 ge,
     scat2(ub, g.L(k + 1, j, i), g.L(k, j, i), 1.0, gz);
 }
 
-// adjoint of Compute_du_center at cell (i, j, k)
-template <class T>
-__device__ void du_center_adj(const Geo &g, T *ub, int i, int j, int k, V3 gc, V3 ge, V3 gz) {
-    const int c = g.L(k, j, i);
-    if (g.nonper(0) && i == g.mx - 2) scat2(ub, c, g.L(k, j, i - 1), 1.0, gc);
-    else if (g.nonper(0) && i == 1) scat2(ub, g.L(k, j, i + 1), c, 1.0, gc);
-    else scat2(ub, g.L(k, j, i + 1), g.L(k, j, i - 1), 0.5, gc);
-    if (g.nonper(1) && j == g.my - 2) scat2(ub, c, g.L(k, j - 1, i), 1.0, ge);
-    else if (g.nonper(1) && j == 1) scat2(ub, g.L(k, j + 1, i), c, 1.0, ge);
-    else scat2(ub, g.L(k, j + 1, i), g.L(k, j - 1, i), 0.5, ge);
-    if (g.nonper(2) && k == g.mz - 2) scat2(ub, c, g.L(k - 1, j, i), 1.0, gz);
-    else if (g.nonper(2) && k == 1) scat2(ub, g.L(k + 1, j, i), c, 1.0, gz);
-    else scat2(ub, g.L(k + 1, j, i), g.L(k - 1, j, i), 0.5, gz);
-}
-
-struct NutBCv { int bc[6]; };
-
-// T: type of the flow fields (ucont, ucat, theta, nu_t) and of their cotangents; P: storage type
-// of the cotangent packets and intermediates (fpbar, nu_eff_bar, the face and cell packets).  The
-// cotangent arithmetic is FP64 in both forms.
+// T: type of the flow fields (ucont, ucat, nu_t) and of their cotangents; P: storage type of what
+// passes between the kernels (fpbar, the nu_eff cotangents, the row sums).  The cotangent arithmetic
+// is FP64 in both forms.
 template <class T, class P>
 struct VjpArgs {
-    const T *ucont, *ucat, *theta, *nut;
+    const T *ucont, *ucat, *nut;
     T *nut_w;           // where k_vjp_pre writes the recomputed nu_t (the array nut reads)
     const double *cs, *rbar;
     const double *csi, *eta, *zet, *icsi, *ieta, *izet, *jcsi, *jeta, *jzet, *kcsi, *keta, *kzet;
     const double *aj, *iaj, *jaj, *kaj;
-    const double *tauI, *tauJ;
     P *fpbar;
     T *vbar, *ubar, *tbar;
     double *csbar;
@@ -133,7 +115,6 @@ struct VjpArgs {
     long n;
     double scale, bscale, tRef, nu;
     int quick, les;
-    int nut_in;         // nu_t is an input array (no |S| path, no Cs)
     int bc_u[6], bc_nut[6];
 };
 
@@ -370,14 +351,15 @@ __device__ __forceinline__ void boundary_face(const VjpArgs<T, P> &A, const Geo 
 // planes, and what goes to the neighbouring rows, `jp` for row j+1, `jm` for row j-1 and (QUICK) `jpp` for row
 // j+2, through LDS where that row is one of the workgroup's four (one barrier a plane) and to memory where it
 // is not: per point the row's own sum `own` and, at the workgroup's ends, jp of its last row, jm of its first,
-// jpp of its last two, on average 5 to 6 values instead of the 36 of three face packets.  k_vjp_finish adds the
+// jpp of its last two, on average 4.5 values (QUICK: 6) instead of the 36 of three face packets.  k_vjp_finish adds the
 // rows.  Buoyancy's theta cotangent comes along, since its icsi.z, jeta.z, kzet.z are loaded here.
 //
-// Bound by memory: 456 bytes a point in FP64 (nine metric vectors 216, row sums 48), about 840 moved, since a wave's 64 points end within cache lines, 4 of them overlap and a chunk of planes loads 3
+// Bound by memory: 456 bytes a point in FP64 (nine metric vectors 216, row sums 48), 755 moved on the hill below
+// (4.2 TB/s), since a wave's 64 points end within cache lines, 4 of them overlap and a chunk of planes loads 3
 // more.  The registers (two waves a SIMD) hold the sums of four planes; the row sums and ucont_bar are
 // written as whole vectors, since stores of 8 of 24 bytes cost a pass over the line each.  Against a launch
 // that wrote the three packets of every face and a cell kernel that gathered them: the adjoint of the
-// 192 x 192 x 128 hill (FP64, QUICK) 2.60 -> 1.49 ms, of which this kernel is 0.84, and of the 384 x 256 x 96
+// 192 x 192 x 128 hill (FP64, QUICK) 2.60 -> 1.48 ms, of which this kernel is 0.84, and of the 384 x 256 x 96
 // box (mixed, central) 3.69 -> 1.94, of which 1.00.  Without the exchange in LDS every row's sums went to
 // memory: 1.52 and 2.06 (this kernel 0.82 and 1.03, k_vjp_finish 0.43 and 0.63 for 0.38 and 0.54); with
 // workgroups of eight rows 1.47 and 1.95, but 0.16 for 0.14 on the 128 x 96 x 64 grid, which they do not fill.
@@ -642,8 +624,8 @@ __device__ __forceinline__ V3 wt3(double w, V3 v) { return V3{w != 0.0 ? w * v.x
 // |S| path of the interior cells (nu_t_bar, Cs_bar, the cotangents of the three du_center vectors), which
 // a workgroup of 8 rows marching along k keeps on chip: along i by lane shifts, along j through LDS (one
 // barrier a plane), along k in the accumulators of three planes.  62 x 6 points a workgroup.
-// Bound by latency: 240 bytes a point in FP64, at 3.0 TB/s; 0.38 ms on the 192 x 192 x 128 hill, 0.54 on the
-// mixed 384 x 256 x 96 box.  Every load of a cell is issued without a branch (with every row's sums read, the
+// Bound by memory and by the latency of its loads: 240 bytes a point in FP64, 368 moved at 4.5 TB/s; 0.38 ms on the
+// 192 x 192 x 128 hill, 0.54 on the mixed 384 x 256 x 96 box.  Every load of a cell is issued without a branch (with every row's sums read, the
 // six faces of nu_t_bar with a condition each took 0.49 and 0.86, 0.43 and 0.62 without); loading the row sums
 // ahead of the barrier as well cost 169 registers for 128 and with them half the waves: 0.50 ms.  The launch
 // bound holds it at 128 (132 of the compiler's own choice would leave three waves a SIMD).
@@ -767,7 +749,7 @@ void vjp_rhs_impl(const Geo &g, const tosca_mesh *mesh, const tosca_params *p, c
     for (int q = 0; q < 3; q++) zero(nueb + q * n, wP, GW + 1);
     TOSCA_LAUNCH("k_vjp_zero", k_vjp_zero_shells, dim3(256, 6, Z.n), dim3(256), 0, s, Z, g);
     VjpArgs<T, P> A;
-    A.ucont = ucont; A.ucat = ucat; A.theta = nullptr; A.cs = cs; A.rbar = rbar;
+    A.ucont = ucont; A.ucat = ucat; A.cs = cs; A.rbar = rbar;
     A.nut = les ? (nut_in ? nut_in : nut) : ucat;
     A.nut_w = nut;
     A.csi = mesh->csi; A.eta = mesh->eta; A.zet = mesh->zet;
@@ -775,7 +757,6 @@ void vjp_rhs_impl(const Geo &g, const tosca_mesh *mesh, const tosca_params *p, c
     A.jcsi = mesh->jcsi; A.jeta = mesh->jeta; A.jzet = mesh->jzet;
     A.kcsi = mesh->kcsi; A.keta = mesh->keta; A.kzet = mesh->kzet;
     A.aj = mesh->aj; A.iaj = mesh->iaj; A.jaj = mesh->jaj; A.kaj = mesh->kaj;
-    A.tauI = p->tau_wall_i; A.tauJ = p->tau_wall_j;
     A.fpbar = fpbar; A.nutbar_acc = nut_bar;
     A.vbar = ucont_bar; A.ubar = ucat_bar; A.tbar = theta_bar; A.csbar = cs_bar;
     for (int q = 0; q < 3; q++) A.nueb[q] = nueb + q * n;
@@ -785,7 +766,6 @@ void vjp_rhs_impl(const Geo &g, const tosca_mesh *mesh, const tosca_params *p, c
     A.scale = scale; A.bscale = buoy_scale; A.tRef = p->t_ref; A.nu = p->nu;
     A.quick = p->div_scheme == TOSCA_DIV_QUICK;
     A.les = les;
-    A.nut_in = nut_in != nullptr;
     for (int q = 0; q < 6; q++) { A.bc_u[q] = p->bc_u[q]; A.bc_nut[q] = p->bc_nut[q]; }
     const bool f32 = sizeof(T) == 4;
     const dim3 cb(64, 4), cg((g.mx - 2 + 63) / 64, (g.my - 2 + 3) / 4, g.mz - 2);
