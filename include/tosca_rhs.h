@@ -490,7 +490,8 @@ typedef struct {
  *     thetaWallFunction faces: the wall heat flux, kappa 0.
  * Then the periodic reset of the face fluxes (resetFacePeriodicFluxesVector).  kt is read for the
  * dynamic models only (may be NULL otherwise); nut whenever LES is active.  Stability-based and
- * structural models (bardinaVreman / bardinaAMD) return TOSCA_ERR_UNSUPPORTED. */
+ * structural models (bardinaVreman / bardinaAMD) return TOSCA_ERR_UNSUPPORTED.  rhs may lie in the
+ * memory of an input, which is read before (the call then copies rhs through the workspace). */
 int tosca_formt(tosca_ctx *ctx, const tosca_mesh *mesh, const tosca_params *params, const tosca_teqn_params *tparams,
                 const double *ucont, const double *theta, const double *nut, const double *kt, double *rhs,
                 double scale, int form_mode);
